@@ -122,7 +122,7 @@ inline int check_option(int option, int64_t value, int num_tiles, std::string* m
         case IDISIM_OPT_GRAPH:
         case IDISIM_OPT_FALLBACK: return IDISIM_OK;
         case IDISIM_OPT_TILE:
-            if (value < -1 || value >= num_tiles) return arg_error(msg, who, "tile variant out of range");
+            if (value < -1 || value >= num_tiles || value == kNumTiles) return arg_error(msg, who, "tile variant out of range");
             if (value == kTileNone) {
                 *msg = std::string(who) + ": tile variant 4 has no kernel";
                 return IDISIM_E_UNSUPPORTED;

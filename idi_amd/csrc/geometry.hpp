@@ -53,6 +53,9 @@ struct Geom {
     // A lane whose own bound T_k = |2 pi (d_k - D_k)| refrho exceeds T / sqrt 2 scales its pair
     // sums by 1 / (1 + T_k^2 / 2 - refc), which keeps the first-order truncation within T^2 / 4.
     float refrho, refc;
+    // Set per launch for the separable tiles: the power of two that brings the largest |r'_cj| to
+    // between 1/2 and 1 (their records are scaled by it, so that FP16 holds the components).
+    float sepscale;
 };
 
 struct Frame {
@@ -203,6 +206,127 @@ __host__ __device__ inline SplitRec make_split_rec(const Geom& g, const Frame& c
     return r;
 }
 
+// Separable tiles: with dq(x, y) = -krev (u_p - u_c) of the pixels of a wave's square about its
+// centre (dx = dy = 0), dq(dx, dy) = dq(dx, 0) + dq(0, dy) + m(dx, dy), and the phasor of a pair is
+// the product of a row and a column phasor but for the mixed remainder m.  r_p = p + dx a + dy b
+// (p the square's centre, a and b the detector axes times the pitch), |r_p|^2 = R^2 (1 + ex + ey +
+// kappa), ex = 2 dx pa + dx^2 aa, ey = 2 dy pb + dy^2 bb, kappa = 2 dx dy ab (0 for orthogonal
+// axes), and with f(e) = (1 + e)^(-1/2)
+//   m = -krev / R (p [f(e) - f(ex) - f(ey) + 1] + dx a [f(e) - f(ex)] + dy b [f(e) - f(ey)]),
+// the brackets as series in e (no cancellation, so FP32 will do; the planner keeps |e| < 0.01).
+// To leading order m = dx dy mu, mu = -krev / R (3 pa pb p - pb a - pa b - ab p).
+struct SepFrame {
+    float p[3], a[3], b[3];  // p / R, a / R, b / R
+    float pa, pb, aa, bb, ab;
+    float mu[3];
+    float krev;
+};
+
+__host__ __device__ inline SepFrame make_sep_frame(const Geom& g, const double r[3])
+{
+    double a[3] = {g.pix, 0.0, 0.0}, b[3] = {0.0, g.pix, 0.0};
+    if (g.rot)
+        for (int i = 0; i < 3; ++i) {
+            a[i] = g.M[3 * i] * g.pix;
+            b[i] = g.M[3 * i + 1] * g.pix;
+        }
+    const double iR2 = 1.0 / (r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+    const double iR = sqrt(iR2);
+    const double pa = (r[0] * a[0] + r[1] * a[1] + r[2] * a[2]) * iR2;
+    const double pb = (r[0] * b[0] + r[1] * b[1] + r[2] * b[2]) * iR2;
+    const double ab = (a[0] * b[0] + a[1] * b[1] + a[2] * b[2]) * iR2;
+    SepFrame f;
+    for (int i = 0; i < 3; ++i) {
+        f.p[i] = (float)(r[i] * iR);
+        f.a[i] = (float)(a[i] * iR);
+        f.b[i] = (float)(b[i] * iR);
+        f.mu[i] = (float)(-g.krev * iR * ((3.0 * pa * pb - ab) * r[i] - pb * a[i] - pa * b[i]));
+    }
+    f.pa = (float)pa;
+    f.pb = (float)pb;
+    f.aa = (float)((a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * iR2);
+    f.bb = (float)((b[0] * b[0] + b[1] * b[1] + b[2] * b[2]) * iR2);
+    f.ab = (float)ab;
+    f.krev = (float)g.krev;
+    return f;
+}
+
+// Two orthonormal directions that hold nearly all of a square's mixed remainder: mu / |mu|, and
+// across it the main direction of the third-order terms
+//   dx^2 dy: -krev / R (...) along -b and p,   dx dy^2: along -a and p,
+// of which the parts across mu span a plane; the larger of the two eigenvectors of their sum of
+// squares.
+__host__ __device__ inline void sep_basis_of(const SepFrame& f, float (&b)[2][3])
+{
+    double e[3] = {f.mu[0], f.mu[1], f.mu[2]};
+    const double n2 = e[0] * e[0] + e[1] * e[1] + e[2] * e[2];
+    const double n = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
+    for (int i = 0; i < 3; ++i) e[i] *= n;
+    if (!(n2 > 0.0)) e[0] = 1.0;
+    // coefficients of dx^2 dy and dx dy^2 in m (over a common factor, at kappa = 0)
+    const double pa = f.pa, pb = f.pb, aa = f.aa, bb = f.bb, inv = 1.0 / (aa + bb + pa * pa + pb * pb);
+    double v[2][3];
+    for (int i = 0; i < 3; ++i) {
+        v[0][i] = (1.5 * aa * pb - 7.5 * pa * pa * pb) * f.p[i] + 3.0 * pa * pb * f.a[i] +
+                  (1.5 * pa * pa - 0.5 * aa) * f.b[i];
+        v[1][i] = (1.5 * bb * pa - 7.5 * pb * pb * pa) * f.p[i] + 3.0 * pa * pb * f.b[i] +
+                  (1.5 * pb * pb - 0.5 * bb) * f.a[i];
+        v[0][i] *= inv;
+        v[1][i] *= inv;
+    }
+    for (int k = 0; k < 2; ++k) {  // across mu
+        const double d = v[k][0] * e[0] + v[k][1] * e[1] + v[k][2] * e[2];
+        for (int i = 0; i < 3; ++i) v[k][i] -= d * e[i];
+    }
+    // the eigenvector (c0, c1) of the larger eigenvalue of the vectors' Gram matrix
+    const double g00 = v[0][0] * v[0][0] + v[0][1] * v[0][1] + v[0][2] * v[0][2];
+    const double g11 = v[1][0] * v[1][0] + v[1][1] * v[1][1] + v[1][2] * v[1][2];
+    const double g01 = v[0][0] * v[1][0] + v[0][1] * v[1][1] + v[0][2] * v[1][2];
+    const double h = 0.5 * (g00 - g11), q = sqrt(h * h + g01 * g01);
+    const double c0 = h >= 0.0 ? h + q : g01, c1 = h >= 0.0 ? g01 : q - h;
+    const double cn = c0 * c0 + c1 * c1 > 0.0 ? 1.0 / sqrt(c0 * c0 + c1 * c1) : 0.0;
+    double w[3], m2 = 0.0;
+    for (int i = 0; i < 3; ++i) {
+        w[i] = cn * (c0 * v[0][i] + c1 * v[1][i]);
+        m2 += w[i] * w[i];
+    }
+    if (!(m2 > 0.0)) {  // any direction across e
+        const int k = fabs(e[0]) < 0.6 ? 0 : (fabs(e[1]) < 0.6 ? 1 : 2);
+        m2 = 0.0;
+        for (int i = 0; i < 3; ++i) {
+            w[i] = (i == k ? 1.0 : 0.0) - e[k] * e[i];
+            m2 += w[i] * w[i];
+        }
+    }
+    const double wn = 1.0 / sqrt(m2);
+    for (int i = 0; i < 3; ++i) {
+        b[0][i] = (float)e[i];
+        b[1][i] = (float)(w[i] * wn);
+    }
+}
+
+// f(e + d) - f(e), f(e) = (1 + e)^(-1/2), to fourth order
+__host__ __device__ inline float sep_df(float e, float d)
+{
+    const float d2 = 3.f * e * (e + d) + d * d;                      // ((e + d)^3 - e^3) / d
+    const float d3 = (2.f * e + d) * (2.f * e * (e + d) + d * d);    // ((e + d)^4 - e^4) / d
+    return d * (-0.5f + 0.375f * (2.f * e + d) - 0.3125f * d2 + 0.2734375f * d3);
+}
+
+// The mixed remainder m(dx, dy) in revolutions per length.
+__host__ __device__ inline void sep_mixed(const SepFrame& f, float dx, float dy, float m[3])
+{
+    const float ex = dx * (2.f * f.pa + dx * f.aa), ey = dy * (2.f * f.pb + dy * f.bb);
+    const float kap = 2.f * dx * dy * f.ab;
+    const float ek = ey + kap;
+    // f(ex + ek) - f(ex) - f(ek) + 1 and f(ek) - f(ey)
+    const float q = ex * ek;
+    float s = q * (0.75f - 0.9375f * (ex + ek) + 1.09375f * (ex * ex + 1.5f * q + ek * ek));
+    s += sep_df(ey, kap);
+    const float cx = dx * sep_df(ex, ek), cy = dy * sep_df(ey, ex + kap);
+    for (int i = 0; i < 3; ++i) m[i] = -f.krev * (s * f.p[i] + cx * f.a[i] + cy * f.b[i]);
+}
+
 // Work item of the persistent batched kernels: one (shot, pixel tile).
 struct WorkItem {
     int32_t shot;
@@ -236,6 +360,10 @@ struct WorkItem {
 // 15: as 14, with the rotation between the two pair centres of a quad (the centring of 7)
 // also taken from the sub-block's reference quad, formed once per emitter and sub-block
 // instead of once per lane: 3 fewer FMA per quad, for a residual the planner tabulates.
+// 17..22 (16 stays unused: the first index past the planner's per-tile tables): the separable tiles of
+// separable.hip, matrix products over the emitters.  A wave owns a rectangle of 32 x 32 (17, 18),
+// 32 x 64 (19, 20) or 16 x 16 pixels (21, 22), a workgroup 2 x 2 of them; the mixed remainder is kept
+// along two directions (17, 19, 21) or in full (18, 20, 22), by 22 to second order.
 constexpr int kNumTiles = 16;
 constexpr int kTileNone = 4;  // reserved index, no kernel
 constexpr int kTilePair1 = 5;
@@ -249,6 +377,20 @@ constexpr int kTileRefC2 = 12;
 constexpr int kTileRefL = 13;
 constexpr int kTileRefS = 14;
 constexpr int kTileRefSC = 15;
+constexpr int kTileSep32 = 17;
+constexpr int kTileSep32V = 18;
+constexpr int kTileSep32W = 19;
+constexpr int kTileSep32WV = 20;
+constexpr int kTileSep16 = 21;
+constexpr int kTileSep16Q = 22;
+constexpr int kNumTilesAll = 23;
+__host__ __device__ constexpr bool tile_sep(int v) { return v >= kTileSep32 && v < kNumTilesAll; }
+// pixels of a wave's rectangle (separable tiles)
+__host__ __device__ constexpr int tile_sep_rows(int v) { return v <= kTileSep32WV ? 32 : 16; }
+__host__ __device__ constexpr int tile_sep_cols(int v)
+{
+    return v == kTileSep32W || v == kTileSep32WV ? 64 : tile_sep_rows(v);
+}
 __host__ __device__ constexpr bool tile_pair(int v) { return v >= kTilePair1 && v <= kTileRefSC; }
 __host__ __device__ constexpr bool tile_pair_centred(int v)
 {
@@ -270,10 +412,13 @@ __host__ __device__ constexpr int tile_ref_order(int v)
     return tile_ref_kind(v) >= 3 ? 1 : tile_ref_kind(v);
 }
 __host__ __device__ constexpr int pair_quads(int v) { return v == kTilePair2 ? 2 : 1; }
-__host__ __device__ constexpr int tile_px(int v) { return v >= 2 && v != kTileNone ? 2 : 1; }
+__host__ __device__ constexpr int tile_px(int v)
+{
+    return tile_sep(v) ? tile_sep_rows(v) / 8 : (v >= 2 && v != kTileNone ? 2 : 1);
+}
 __host__ __device__ constexpr int tile_py(int v)
 {
-    return v == 0 || v == kTileNone ? 1 : (v == 3 || v == kTilePair2 || v == kTileBlock ? 4 : 2);
+    return tile_sep(v) ? tile_sep_cols(v) / 8 : v == 0 || v == kTileNone ? 1 : (v == 3 || v == kTilePair2 || v == kTileBlock ? 4 : 2);
 }
 __host__ __device__ constexpr int tile_rows(int v) { return 16 * tile_px(v); }
 __host__ __device__ constexpr int tile_cols(int v) { return 16 * tile_py(v); }

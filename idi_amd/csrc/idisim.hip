@@ -53,10 +53,11 @@ int fail(int code, const std::string& msg)
 // larger emitter extent can push a tile's error bound past the tolerance).
 struct TuneKey {
     int kind, has_amp, batched, split_path, nbucket;
+    int sep;  // the separable tiles were candidates
     bool operator<(const TuneKey& o) const
     {
-        return std::tie(kind, has_amp, batched, split_path, nbucket) <
-               std::tie(o.kind, o.has_amp, o.batched, o.split_path, o.nbucket);
+        return std::tie(kind, has_amp, batched, split_path, nbucket, sep) <
+               std::tie(o.kind, o.has_amp, o.batched, o.split_path, o.nbucket, o.sep);
     }
 };
 
@@ -217,6 +218,13 @@ Geom split_geom(const idisim_handle* h, int tile, bool* w)
         gl.refrho = (float)(h->rho * (1.0 + sigma_bound(h, tile, h->rho)));
         gl.refc = (float)ref_trunc_centre(h, tile, h->rho);
     }
+    if (tile_sep(tile)) {
+        const double r = h->rho * (1.0 + sigma_bound(h, tile, h->rho));
+        int ex = 0;
+        if (r > 0.0 && std::isfinite(r)) (void)std::frexp(r, &ex);
+        // 2^-ex and its inverse stay normal FP32 numbers; emitters all at the origin have no scale
+        gl.sepscale = (float)std::ldexp(1.0, -std::min(std::max(ex, -120), 120));
+    }
     return gl;
 }
 
@@ -230,6 +238,7 @@ struct FwdCall {
     hipStream_t st;
     bool split_path;  // FP32-split kernels (false: FP64 kernels)
     bool out_f32;     // FP64 kernels writing a complex64 / float32 output (fallback)
+    bool sep = false; // the separable tiles are the candidates (use_sep_tiles)
     // fixed device scratch of idisim_forward_noalloc (nullptr: the handle's own, grown on demand)
     void* fixed = nullptr;
     size_t fixed_cap = 0;
@@ -301,6 +310,10 @@ int run_forward(idisim_handle* h, const FwdCall& c, int tile, int splits)
             const float* tab = nullptr;
             if (int rc = pair_table(h, c, tile, &tab)) return rc;
             IDISIM_HIP(launch_fwd_pair(tile, a, gl, c.emit, c.amp, c.n, splits, tab, partial, c.out, c.kind, c.st));
+        } else if (tile_sep(tile)) {
+            if (h->summode != 0) return fail(IDISIM_E_UNSUPPORTED, "the separable tiles have no per-term Kahan mode");
+            if (w) return fail(IDISIM_E_UNSUPPORTED, "the separable tiles need the curvature folded into A");
+            IDISIM_HIP(launch_fwd_sep(tile, a, gl, c.emit, c.amp, c.n, splits, partial, c.out, c.kind, c.st));
         } else {
             IDISIM_HIP(launch_fwd_split(tile, w, a, h->summode, gl, c.emit, c.amp, c.n, splits, partial, c.out,
                                         c.kind, c.st));
@@ -338,6 +351,38 @@ int run_forward_partials(idisim_handle* h, const FwdCall& c, int tile, int split
     return IDISIM_OK;
 }
 
+// The separable tiles take a forward of at least kSepPairs emitter-pixel pairs (n rounded down to its
+// tuning bucket) where they meet the bound.  Intensities: from 1e8 on (1000 emitters on 128 x 128
+// pixels, 1.6e7 pairs, take 13 to 14 us either way; 2048 on 256 x 256, 1.3e8 pairs, 22 against 34 us;
+// 12345 on 333 x 211 79 against 144; 100000 on 512 x 512 1.07 against 3.29 ms).  Fields: from 5e8 on.
+// Between the two lines they would be faster as well (4096 on 256 x 256: 30 against 52 us), but a field
+// there stays on the tiles that idisim_loss_grad_l2 sums its loss from, so that it and
+// idisim_adjoint_l2 on it give that call's bits at the sizes of a fit: the FP64 loss follows the
+// field's rounding, and the loss must not change.
+constexpr double kSepPairsIntensity = 1e8, kSepPairsField = 5e8;
+
+// The separable candidates of a call in `tiles`, in place of the others: of each rectangle the one
+// with the fewest sums.
+bool use_sep_tiles(const idisim_handle* h, int64_t n, int kind, bool split_path, std::vector<int>* tiles)
+{
+    if (!split_path || h->force_tile >= 0) return false;
+    const double pairs = std::ldexp(1.0, nbucket(n)) * (double)h->g.n0 * (double)h->g.n1;
+    if (pairs < (kind == OUT_INTENSITY ? kSepPairsIntensity : kSepPairsField)) return false;
+    std::vector<int> sep;
+    for (int v : eligible_sep_tiles(h, h->rho))
+        if (sep.empty() || sep_shape(v) != sep_shape(sep.back())) sep.push_back(v);
+    if (sep.empty()) return false;
+    *tiles = sep;
+    return true;
+}
+
+// Workgroups per CU that a heuristic split aims at: as many as are resident of the separable tiles.
+int64_t target_groups(const idisim_handle* h, int tile)
+{
+    const int per_cu = !tile_sep(tile) ? 4 : (tile_sep_cols(tile) == 64 ? 1 : (tile_sep_rows(tile) == 32 ? 2 : 4));
+    return (int64_t)per_cu * h->num_cus;
+}
+
 std::vector<int> split_candidates(const idisim_handle* h, int64_t n, int tile)
 {
     const int64_t maxs = std::max<int64_t>(1, (n + kSplitGrain - 1) / kSplitGrain);
@@ -359,7 +404,7 @@ int heuristic_split(const idisim_handle* h, int64_t n, int tile)
     const int tiles = ((h->g.n0 + tile_rows(tile) - 1) / tile_rows(tile)) *
                       ((h->g.n1 + tile_cols(tile) - 1) / tile_cols(tile));
     for (int s : c)
-        if ((int64_t)tiles * s >= 4LL * h->num_cus) return s;
+        if ((int64_t)tiles * s >= target_groups(h, tile)) return s;
     return c.back();
 }
 
@@ -367,7 +412,7 @@ int heuristic_split(const idisim_handle* h, int64_t n, int tile)
 // candidate forwards into c.out), or the heuristic.
 int plan_choose(idisim_handle* h, const FwdCall& c, const std::vector<int>& tiles, Choice& ch)
 {
-    const TuneKey key{c.kind, c.amp != nullptr, 0, c.split_path ? 1 : 0, nbucket(c.n)};
+    const TuneKey key{c.kind, c.amp != nullptr, 0, c.split_path ? 1 : 0, nbucket(c.n), c.sep ? 1 : 0};
     auto it = h->tuned.find(key);
     const bool forced = h->force_tile >= 0 || h->force_split > 0;
     if (forced) {
@@ -449,9 +494,19 @@ int plan_choose(idisim_handle* h, const FwdCall& c, const std::vector<int>& tile
             }
         }
     } else {
-        // heuristic: a mirror-pair quad per lane if allowed, enough splits for 4 WG/CU
-        ch.tile = tiles.front();
-        for (int v : {kTileRefL, kTileRef1, kTileRefC1, kTileRefSC, kTileRefS, kTileRef2, kTileRefC2, kTilePair1, kTileBlock, kTilePairC, 2, 1, 3, 0})
+        // heuristic: a mirror-pair quad per lane if allowed (of the separable tiles the widest that can
+        // fill the device), enough splits for 4 WG/CU (or all that are resident)
+        ch.tile = c.sep ? tiles.back() : tiles.front();
+        if (c.sep) {
+            for (int v : tiles) {
+                const int64_t wgs = (int64_t)((h->g.n0 + tile_rows(v) - 1) / tile_rows(v)) *
+                                    ((h->g.n1 + tile_cols(v) - 1) / tile_cols(v)) * ((c.n + kChunk - 1) / kChunk);
+                if (wgs >= 2 * target_groups(h, v)) {
+                    ch.tile = v;
+                    break;
+                }
+            }
+        } else for (int v : {kTileRefL, kTileRef1, kTileRefC1, kTileRefSC, kTileRefS, kTileRef2, kTileRefC2, kTilePair1, kTileBlock, kTilePairC, 2, 1, 3, 0})
             if (has_tile(tiles, v)) {
                 ch.tile = v;
                 break;
@@ -552,6 +607,8 @@ int launch_batched(idisim_handle* h, const BatchCall& c, int tile, int blocks_pe
             if (w) return fail(IDISIM_E_UNSUPPORTED, "the mirror-pair tiles need the curvature folded into A");
             IDISIM_HIP(launch_batched_pair(tile, a, gl, c.emit, c.amp, h->d_items, h->nitems, h->d_counter, nblocks,
                                            c.out, c.kind, st));
+        } else if (tile_sep(tile)) {
+            return fail(IDISIM_E_UNSUPPORTED, "the separable tiles have no batched kernel");
         } else {
             IDISIM_HIP(launch_batched_split(tile, w, a, h->summode, gl, c.emit, c.amp, h->d_items, h->nitems,
                                             h->d_counter, nblocks, c.out, c.kind, st));
@@ -743,6 +800,7 @@ int idisim_create(idisim_handle** out, const idisim_geometry* geom, int precisio
         h->num_cus = prop.multiProcessorCount;
     h->g = make_geom(*geom);
     planner_tables(h);
+    planner_sep_tables(h);
     h->plan.precision = precision;
     if (hipHostMalloc(reinterpret_cast<void**>(&h->h_viol), sizeof(unsigned int),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
@@ -792,7 +850,7 @@ int idisim_set_option(idisim_handle* h, int option, int64_t value)
 {
     if (!h) return fail(IDISIM_E_INVALID, "idisim_set_option: NULL handle");
     std::string msg;
-    if (int rc = check_option(option, value, kNumTiles, &msg)) return fail(rc, msg);
+    if (int rc = check_option(option, value, kNumTilesAll, &msg)) return fail(rc, msg);
     switch (option) {
         case IDISIM_OPT_AUTOTUNE: h->autotune = value ? 1 : 0; break;
         case IDISIM_OPT_TILE: h->force_tile = (int)value; break;
@@ -1027,7 +1085,7 @@ static int forward_call(idisim_handle* h, const double* emitters, const double* 
     rc = choose_path(h, rho, &tiles, &split_path);
     if (rc) return rc;
     FwdCall c{emitters, amplitudes, n, out, out_kind, st, split_path,
-              h->precision == IDISIM_PREC_FP32SPLIT && !split_path};
+              h->precision == IDISIM_PREC_FP32SPLIT && !split_path, use_sep_tiles(h, n, out_kind, split_path, &tiles)};
     if (noalloc) {
         c.fixed = h->noalloc;
         c.fixed_cap = IDISIM_NOALLOC_SCRATCH_BYTES;
@@ -1102,7 +1160,7 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
     BatchCall c{emitters, amplitudes, out, out_kind, st, split_path};
 
     const TuneKey key{out_kind, amplitudes != nullptr, 1, split_path ? 1 : 0,
-                      nbucket(std::max<int64_t>(1, total / nshots))};
+                      nbucket(std::max<int64_t>(1, total / nshots)), 0};
     Choice ch;
     auto it = h->tuned.find(key);
     if (h->force_tile >= 0 || h->force_split > 0) {

@@ -29,8 +29,8 @@ struct Planner {
     Geom g{};
     double tol_rev = 5e-6;  // per-term phase tolerance
     int summode = 0;        // 1: Kahan on every term (the mirror-pair tiles have no such mode)
-    double du_max[kNumTiles] = {};
-    double dR_max[kNumTiles] = {};
+    double du_max[kNumTilesAll] = {};
+    double dR_max[kNumTilesAll] = {};
     double Rmin = 0.0, Rmax = 0.0;
     double pair_coef = 0.0;   // mirror-pair remainder per unit emitter extent (rev per length)
     double block_coef = 0.0;  // bound of |m_k - m_1| of the 2 x 4 block pairs per unit extent
@@ -38,7 +38,17 @@ struct Planner {
     double refs_coef = 0.0;   // the same against the 8 x 8 pixel sub-block reference (variants 14, 15)
     double cent_coef = 0.0;   // largest |(m_0 - m_1) - (m_0 - m_1) of the sub-block reference| (variant 15)
     double lin_coef = 0.0;    // largest residual of the linear wave reference (variant 13) per unit extent
+    // separable tiles, wave rectangles of 32 x 32 (0), 32 x 64 (1) and 16 x 16 (2) pixels: the largest
+    // row or column phase, the largest mixed remainder |m|, its largest part beyond dx dy mu and beyond
+    // the two directions of sep_basis_of, per unit extent (rev per length)
+    double sep_line_max[3] = {}, sep_mixed_max[3] = {}, sep_rest_max[3] = {}, sep_off_max[3] = {};
 };
+
+// The truncation (revolutions) that a separable tile may leave.  Its relative L2 error is about a
+// twelfth of the bound in radians (the bound is reached at a tile's corner by an emitter at the
+// extent), so 7e-7 at most and 2e-7 at 1.3e-6 over the corner tile of a 512 x 512 image: with it images
+// are as accurate as with the mirror-pair tiles.
+constexpr double kSepTruncRev = 1.4e-6;
 
 inline void planner_tables(Planner* h)
 {
@@ -202,6 +212,81 @@ inline void planner_tables(Planner* h)
     }
 }
 
+inline int sep_shape(int v) { return tile_sep_rows(v) == 16 ? 2 : (tile_sep_cols(v) == 64 ? 1 : 0); }
+
+// The separable tiles' tables: the extent of their workgroup tiles (2 x 2 rectangles, whole also
+// where the detector ends inside one), and for every rectangle the row and column phases at its edges
+// and the mixed remainder at its corners, where they are largest (dx dy to leading order), each with
+// 5% margin; infinite where the remainder's series would not hold (|e| >= 0.01) and above
+// 2048 x 2048 pixels.
+inline void planner_sep_tables(Planner* h)
+{
+    const Geom& g = h->g;
+    const double inf = std::numeric_limits<double>::infinity();
+    for (int t = 0; t < 3; ++t) {
+        const int TX = t == 2 ? 16 : 32, TY = t == 1 ? 64 : TX;
+        const double hx = 0.5 * (TX - 1), hy = 0.5 * (TY - 1);
+        double line = 0.0, worst = 0.0, rest = 0.0, off = 0.0, du = 0.0, dR = 0.0;
+        bool ok = (int64_t)g.n0 * g.n1 <= (int64_t)2048 * 2048;
+        for (int x0 = 0; x0 < g.n0 && ok; x0 += TX) {
+            for (int y0 = 0; y0 < g.n1 && ok; y0 += TY) {
+                const double cx = x0 + hx, cy = y0 + hy;
+                double r[3];
+                pixel_pos(g, cx, cy, r);
+                const Frame c = make_frame(r);
+                const SepFrame sf = make_sep_frame(g, r);
+                const double e = hx * (2.0 * std::fabs((double)sf.pa) + hx * (double)sf.aa) +
+                                 hy * (2.0 * std::fabs((double)sf.pb) + hy * (double)sf.bb) +
+                                 2.0 * hx * hy * std::fabs((double)sf.ab);
+                ok = e < 0.01;
+                float b[2][3];
+                sep_basis_of(sf, b);
+                const Frame wc = pixel_frame(g, x0 / (2 * TX) * (2 * TX) + TX - 0.5, y0 / (2 * TY) * (2 * TY) + TY - 0.5);
+                const Frame fx[2] = {pixel_frame(g, cx - hx, cy), pixel_frame(g, cx + hx, cy)};
+                const Frame fy[2] = {pixel_frame(g, cx, cy - hy), pixel_frame(g, cx, cy + hy)};
+                for (int i = 0; i < 2; ++i) {
+                    for (int j = 0; j < 2; ++j) {
+                        const Frame f = pixel_frame(g, cx + (2 * i - 1) * hx, cy + (2 * j - 1) * hy);
+                        const double dd = (2 * i - 1) * (2 * j - 1) * hx * hy;
+                        double m[3], u2 = 0.0, m2 = 0.0, s2 = 0.0, o2 = 0.0, m0 = 0.0, m1 = 0.0, lx = 0.0, ly = 0.0;
+                        for (int k = 0; k < 3; ++k) {
+                            const double dx = g.krev * (fx[i].u[k] - c.u[k]), dy = g.krev * (fy[j].u[k] - c.u[k]);
+                            m[k] = -g.krev * ((f.u[k] - fx[i].u[k]) - (fy[j].u[k] - c.u[k]));
+                            const double s = m[k] - dd * (double)sf.mu[k];
+                            u2 += (f.u[k] - wc.u[k]) * (f.u[k] - wc.u[k]);
+                            lx += dx * dx;
+                            ly += dy * dy;
+                            m2 += m[k] * m[k];
+                            s2 += s * s;
+                            m0 += m[k] * (double)b[0][k];
+                            m1 += m[k] * (double)b[1][k];
+                        }
+                        for (int k = 0; k < 3; ++k) {
+                            const double o = m[k] - m0 * (double)b[0][k] - m1 * (double)b[1][k];
+                            o2 += o * o;
+                        }
+                        du = std::max(du, std::sqrt(u2));
+                        dR = std::max(dR, std::fabs(f.R - wc.R));
+                        line = std::max(line, std::sqrt(std::max(lx, ly)));
+                        worst = std::max(worst, std::sqrt(m2));
+                        rest = std::max(rest, std::sqrt(s2));
+                        off = std::max(off, std::sqrt(o2));
+                    }
+                }
+            }
+        }
+        h->sep_line_max[t] = 1.05 * line;
+        h->sep_mixed_max[t] = ok ? 1.05 * worst : inf;
+        h->sep_rest_max[t] = ok ? 1.05 * rest : inf;
+        h->sep_off_max[t] = ok ? 1.05 * off : inf;
+        for (int v = kTileSep32; v < kNumTilesAll; ++v) {
+            if (sep_shape(v) != t) continue;
+            h->du_max[v] = 1.05 * du;
+            h->dR_max[v] = 1.05 * dR;
+        }
+    }
+}
+
 // Error (revolutions) of folding W_cj into A_cj, i.e. of replacing lam_p W_cj
 // by W_cj: W_max max|lam_p - 1|.
 inline double fold_error(const Planner* h, int v, double rho)
@@ -249,6 +334,21 @@ inline double ref_trunc_centre(const Planner* h, int v, double rho)
     return std::isfinite(T) ? 0.25 * T * T : 0.0;
 }
 
+// What the separable tile v drops (revolutions) for emitters within |r_j| <= rho: with M the largest
+// mixed phase 2 pi m . r' (rad), (1 + i M) leaves M^2 / 2, and with two directions the part of m
+// across both besides; the second-order term of kTileSep16Q, taken along mu, leaves M^3 / 6 and M
+// times the part of m beyond dx dy mu.
+inline double sep_trunc(const Planner* h, int v, double rho)
+{
+    const int t = sep_shape(v);
+    const double r = kTwoPi * rho * (1.0 + sigma_bound(h, v, rho));
+    const double M = h->sep_mixed_max[t] * r;
+    if (!std::isfinite(M)) return std::numeric_limits<double>::infinity();
+    if (v == kTileSep16Q) return (M * M * M / 6.0 + M * h->sep_rest_max[t] * r) * kInv2Pi;
+    const double off = v == kTileSep32V || v == kTileSep32WV ? 0.0 : h->sep_off_max[t] * r;
+    return (0.5 * M * M + off) * kInv2Pi;
+}
+
 // A-priori bound of the per-term phase error (revolutions) of tile variant v
 // for emitters within |r_j| <= rho.
 inline double plan_bound(const Planner* h, int v, double rho)
@@ -264,13 +364,22 @@ inline double plan_bound(const Planner* h, int v, double rho)
     if (g.nf || g.secondorder) wmax = rho * rho / (2.0 * Rlo);
     const double W = g.krev * wmax;
     const double B = g.krev * ds * (1.0 + sig);
-    const double tau = 0.5 + W + B;
-    const double ulp = std::ldexp(1.0, std::ilogb(tau) - 23);
     const double u24 = std::ldexp(1.0, -24);
-    double e = 2.0 * ulp;                // four FMA roundings of tau, each <= ulp/2
-    e += 2.0 * u24 * B;                  // dq and r' rounded to FP32: sum_i |dq_i r_i| <= B
-    e += 0.5 * u24 + 6.0 * u24 * W;      // A rounded; W formed in FP32; lam rounded
-    e += 4.0 * u24 * B;                  // r' = r (1 + sigma) formed in FP32
+    double e = 0.0;
+    if (tile_sep(v)) {
+        // the row phase about the wave's centre, whose A is reduced in FP64 and rounded (|tau| <= 1/2 + L,
+        // three FMA), the column phase within L (three), each with dq and r' rounded
+        const double L = h->sep_line_max[sep_shape(v)] * rho * (1.0 + sig);
+        e += 1.5 * std::ldexp(1.0, std::ilogb(0.5 + L) - 23) + 3.0 * u24 * L + 12.0 * u24 * L + 0.5 * u24 +
+             6.0 * u24 * W;
+    } else {
+        const double tau = 0.5 + W + B;
+        const double ulp = std::ldexp(1.0, std::ilogb(tau) - 23);
+        e += 2.0 * ulp;                // four FMA roundings of tau, each <= ulp/2
+        e += 2.0 * u24 * B;            // dq and r' rounded to FP32: sum_i |dq_i r_i| <= B
+        e += 0.5 * u24 + 6.0 * u24 * W;  // A rounded; W formed in FP32; lam rounded
+        e += 4.0 * u24 * B;            // r' = r (1 + sigma) formed in FP32
+    }
     if (g.nf) {
         const double R3 = Rlo * Rlo * Rlo;
         const double wss = Rhi * Rhi / R3;
@@ -285,8 +394,18 @@ inline double plan_bound(const Planner* h, int v, double rho)
     const double fe = fold_error(h, v, rho);
     if (fe <= 0.1 * h->tol_rev) {
         e += fe;  // W folded into A
-    } else if (tile_pair(v) && (g.nf || g.secondorder)) {
+    } else if ((tile_pair(v) || tile_sep(v)) && (g.nf || g.secondorder)) {
         return std::numeric_limits<double>::infinity();  // mirror pairs need the fold
+    }
+    if (tile_sep(v)) {
+        // a second sincos; the phasors split into two FP16 parts each (2^-23 per component, the product
+        // of the low parts dropped); the mixed terms in FP16 (four factors rounded to 2^-11 of at most
+        // M); r' = r (1 + sigma) in FP32 also in the phase of the wave's centre
+        const double trunc = sep_trunc(h, v, rho);
+        if (!(trunc <= kSepTruncRev)) return std::numeric_limits<double>::infinity();
+        const double M = kTwoPi * h->sep_mixed_max[sep_shape(v)] * rho * (1.0 + sig);
+        e += kSinCosErrRev + 4.0 * u24 * B + trunc + (M * 0x1p-9 + 12.0 * u24) * kInv2Pi;
+        return e;
     }
     if (tile_pair(v)) {
         const double rem = h->pair_coef * rho * (1.0 + sig);  // |e_k| = |(m_k - mc) . r'|
@@ -338,6 +457,15 @@ inline std::vector<int> eligible_tiles(const Planner* h, double rho, double* bes
         *best_bound = std::min(*best_bound, b);
         if (b <= h->tol_rev) out.push_back(v);
     }
+    return out;
+}
+
+// The separable tiles that meet the tolerance, the widest first.
+inline std::vector<int> eligible_sep_tiles(const Planner* h, double rho)
+{
+    std::vector<int> out;
+    for (int v : {kTileSep32W, kTileSep32WV, kTileSep32, kTileSep32V, kTileSep16, kTileSep16Q})
+        if (h->summode == 0 && plan_bound(h, v, rho) <= h->tol_rev) out.push_back(v);
     return out;
 }
 
