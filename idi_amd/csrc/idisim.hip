@@ -363,17 +363,22 @@ constexpr double kSepPairsIntensity = 1e8, kSepPairsField = 5e8;
 
 // The separable candidates of a call in `tiles`, in place of the others: of each rectangle the one
 // with the fewest sums.
-bool use_sep_tiles(const idisim_handle* h, int64_t n, int kind, bool split_path, std::vector<int>* tiles)
+bool sep_candidates(const idisim_handle* h, std::vector<int>* tiles)
 {
-    if (!split_path || h->force_tile >= 0) return false;
-    const double pairs = std::ldexp(1.0, nbucket(n)) * (double)h->g.n0 * (double)h->g.n1;
-    if (pairs < (kind == OUT_INTENSITY ? kSepPairsIntensity : kSepPairsField)) return false;
     std::vector<int> sep;
     for (int v : eligible_sep_tiles(h, h->rho))
         if (sep.empty() || sep_shape(v) != sep_shape(sep.back())) sep.push_back(v);
     if (sep.empty()) return false;
     *tiles = sep;
     return true;
+}
+
+bool use_sep_tiles(const idisim_handle* h, int64_t n, int kind, bool split_path, std::vector<int>* tiles)
+{
+    if (!split_path || h->force_tile >= 0) return false;
+    const double pairs = std::ldexp(1.0, nbucket(n)) * (double)h->g.n0 * (double)h->g.n1;
+    if (pairs < (kind == OUT_INTENSITY ? kSepPairsIntensity : kSepPairsField)) return false;
+    return sep_candidates(h, tiles);
 }
 
 // Workgroups per CU that a heuristic split aims at: as many as are resident of the separable tiles.
@@ -590,6 +595,7 @@ struct BatchCall {
     int kind;
     hipStream_t st;
     bool split_path;
+    bool sep = false;  // the separable tiles are the candidates
 };
 
 int launch_batched(idisim_handle* h, const BatchCall& c, int tile, int blocks_per_cu, hipStream_t st)
@@ -608,7 +614,10 @@ int launch_batched(idisim_handle* h, const BatchCall& c, int tile, int blocks_pe
             IDISIM_HIP(launch_batched_pair(tile, a, gl, c.emit, c.amp, h->d_items, h->nitems, h->d_counter, nblocks,
                                            c.out, c.kind, st));
         } else if (tile_sep(tile)) {
-            return fail(IDISIM_E_UNSUPPORTED, "the separable tiles have no batched kernel");
+            if (h->summode != 0) return fail(IDISIM_E_UNSUPPORTED, "the separable tiles have no per-term Kahan mode");
+            if (w) return fail(IDISIM_E_UNSUPPORTED, "the separable tiles need the curvature folded into A");
+            IDISIM_HIP(launch_batched_sep(tile, a, gl, c.emit, c.amp, h->d_items, h->nitems, h->d_counter, nblocks,
+                                          c.out, c.kind, st));
         } else {
             IDISIM_HIP(launch_batched_split(tile, w, a, h->summode, gl, c.emit, c.amp, h->d_items, h->nitems,
                                             h->d_counter, nblocks, c.out, c.kind, st));
@@ -626,6 +635,7 @@ int occupancy(idisim_handle* h, const BatchCall& c, int tile)
     if (c.split_path) {
         const bool w = (g.nf || g.secondorder) && fold_error(h, tile, h->rho) > 0.1 * h->tol_rev;
         if (tile_pair(tile)) return occupancy_batched_pair(tile, (c.amp != nullptr) || (g.nf && g.scale));
+        if (tile_sep(tile)) return occupancy_batched_sep(tile, (c.amp != nullptr) || (g.nf && g.scale));
         return occupancy_batched_split(tile, w, (c.amp != nullptr) || (g.nf && g.scale), h->summode);
     }
     return occupancy_batched_fp64(tile);
@@ -1158,9 +1168,15 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
         return IDISIM_OK;
     }
     BatchCall c{emitters, amplitudes, out, out_kind, st, split_path};
+    // the separable tiles from 1e8 pairs on: 40 shots of 20 to 60 emitters take 48 against 45 us on
+    // 128 x 128 pixels (2.6e7 pairs) and 52 against 64 us on 256 x 256 (1e8); 64 shots of 1000 to 50000 on
+    // 256 x 256 8.6 against 16.3 ms
+    if (split_path && h->force_tile < 0 &&
+        (double)total * (double)h->g.n0 * (double)h->g.n1 >= kSepPairsIntensity)
+        c.sep = sep_candidates(h, &tiles);
 
     const TuneKey key{out_kind, amplitudes != nullptr, 1, split_path ? 1 : 0,
-                      nbucket(std::max<int64_t>(1, total / nshots)), 0};
+                      nbucket(std::max<int64_t>(1, total / nshots)), c.sep ? 1 : 0};
     Choice ch;
     auto it = h->tuned.find(key);
     if (h->force_tile >= 0 || h->force_split > 0) {
@@ -1171,22 +1187,18 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
     } else if (it != h->tuned.end() && has_tile(tiles, it->second.tile)) {
         ch = it->second;
     } else if (h->autotune) {
-        // time the candidates on a prefix of the batch of at most ~2e11 pairs (2e10 for the
-        // FP64 kernels); a shot that crosses the cap is cut
-        const double npix = (double)h->g.n0 * (double)h->g.n1;
+        // time the candidates on at most ~2e11 pairs (2e10 for the FP64 kernels), every shot cut to the
+        // same share: the queue keeps its number of items, on which the choice depends (two shots of 1e6
+        // emitters on 1024 x 1024 pixels are 512 items of 64 x 64 pixels or 256 of 64 x 128)
         const double cap = split_path ? 2e11 : 2e10;
-        std::vector<int64_t> toff(1, 0);
-        for (int64_t s = 0; s < nshots; ++s) {
-            int64_t end = offsets[s + 1];
-            const double before = (double)offsets[s] * npix;
-            if (before + (double)(end - offsets[s]) * npix > cap) {
-                const int64_t room = std::max<int64_t>(kChunk, (int64_t)((cap - before) / npix));
-                toff.push_back(std::min(end, offsets[s] + room));
-                break;
+        const double share = std::min(1.0, cap / ((double)total * (double)h->g.n0 * (double)h->g.n1));
+        std::vector<int64_t> toff(offsets, offsets + nshots + 1);
+        if (share < 1.0)
+            for (int64_t s = 1; s <= nshots; ++s) {
+                const int64_t ns = offsets[s] - offsets[s - 1];
+                toff[s] = toff[s - 1] + std::min(ns, std::max<int64_t>((int64_t)(share * (double)ns), kChunk));
             }
-            toff.push_back(end);
-        }
-        const int64_t tshots = (int64_t)toff.size() - 1;
+        const int64_t tshots = nshots;
         Timer tm;
         double best = std::numeric_limits<double>::infinity();
         for (int v : tiles) {
@@ -1194,7 +1206,7 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
             if (rc) return rc;
             const int occ = occupancy(h, c, v);
             std::vector<int> bpcs = {occ};
-            if (occ > 2) bpcs.push_back(occ / 2);
+            if (occ > 1) bpcs.push_back(occ / 2);  // fewer at a time balance a queue of few items better
             for (int bpc : bpcs) {
                 rc = launch_batched(h, c, v, bpc, st);  // warm-up
                 if (rc) return rc;
@@ -1215,12 +1227,15 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
         }
         h->tuned[key] = ch;
     } else {
-        ch.tile = tiles.front();
-        for (int v : {kTileRefL, kTileRef1, kTileRefC1, kTileRefSC, kTileRefS, kTileRef2, kTileRefC2, kTilePair1, kTileBlock, kTilePairC, 2, 1, 3, 0})
-            if (has_tile(tiles, v)) {
-                ch.tile = v;
-                break;
-            }
+        ch.tile = c.sep ? tiles.back() : tiles.front();
+        if (!c.sep) {
+            for (int v : {kTileRefL, kTileRef1, kTileRefC1, kTileRefSC, kTileRefS, kTileRef2, kTileRefC2, kTilePair1,
+                          kTileBlock, kTilePairC, 2, 1, 3, 0})
+                if (has_tile(tiles, v)) {
+                    ch.tile = v;
+                    break;
+                }
+        }
         ch.split = occupancy(h, c, ch.tile);
     }
     rc = build_items(h, offsets, nshots, ch.tile, st);

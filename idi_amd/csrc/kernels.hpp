@@ -73,6 +73,10 @@ int occupancy_batched_pair(int v, bool a);
 // Separable tiles (tile_sep(v)): g.sepscale set, W folded into A as for the mirror-pair tiles.
 hipError_t launch_fwd_sep(int v, bool a, const Geom& g, const double* emit, const double* amp, int64_t n, int splits,
                           float4* partial, void* out, int kind, hipStream_t st);
+hipError_t launch_batched_sep(int v, bool a, const Geom& g, const double* emit, const double* amp,
+                              const WorkItem* items, int nitems, int* counter, int nblocks, void* out, int kind,
+                              hipStream_t st);
+int occupancy_batched_sep(int v, bool a);
 
 // Literal FP64 forward.
 hipError_t launch_fwd_fp64(int v, const Geom& g, const double* emit, const double* amp, int64_t n, int splits,

@@ -39,7 +39,7 @@ struct Planner {
     double cent_coef = 0.0;   // largest |(m_0 - m_1) - (m_0 - m_1) of the sub-block reference| (variant 15)
     double lin_coef = 0.0;    // largest residual of the linear wave reference (variant 13) per unit extent
     // separable tiles, wave rectangles of 32 x 32 (0), 32 x 64 (1) and 16 x 16 (2) pixels: the largest
-    // row or column phase, the largest mixed remainder |m|, its largest part beyond dx dy mu and beyond
+    // column phase, the largest mixed remainder |m|, its largest part beyond dx dy mu and beyond
     // the two directions of sep_basis_of, per unit extent (rev per length)
     double sep_line_max[3] = {}, sep_mixed_max[3] = {}, sep_rest_max[3] = {}, sep_off_max[3] = {};
 };
@@ -267,7 +267,7 @@ inline void planner_sep_tables(Planner* h)
                         }
                         du = std::max(du, std::sqrt(u2));
                         dR = std::max(dR, std::fabs(f.R - wc.R));
-                        line = std::max(line, std::sqrt(std::max(lx, ly)));
+                        line = std::max(line, std::sqrt(ly));
                         worst = std::max(worst, std::sqrt(m2));
                         rest = std::max(rest, std::sqrt(s2));
                         off = std::max(off, std::sqrt(o2));
@@ -367,10 +367,10 @@ inline double plan_bound(const Planner* h, int v, double rho)
     const double u24 = std::ldexp(1.0, -24);
     double e = 0.0;
     if (tile_sep(v)) {
-        // the row phase about the wave's centre, whose A is reduced in FP64 and rounded (|tau| <= 1/2 + L,
-        // three FMA), the column phase within L (three), each with dq and r' rounded
+        // the row phase (|tau| <= 1/2 + W + B, three FMA) and the column phase (within L, three), dq rounded
+        // in both and r' = r (1 + sigma) formed in FP32 (their sum is within B)
         const double L = h->sep_line_max[sep_shape(v)] * rho * (1.0 + sig);
-        e += 1.5 * std::ldexp(1.0, std::ilogb(0.5 + L) - 23) + 3.0 * u24 * L + 12.0 * u24 * L + 0.5 * u24 +
+        e += 1.5 * std::ldexp(1.0, std::ilogb(0.5 + W + B) - 23) + 3.0 * u24 * L + 6.0 * u24 * B + 0.5 * u24 +
              6.0 * u24 * W;
     } else {
         const double tau = 0.5 + W + B;
@@ -399,12 +399,15 @@ inline double plan_bound(const Planner* h, int v, double rho)
     }
     if (tile_sep(v)) {
         // a second sincos; the phasors split into two FP16 parts each (2^-23 per component, the product
-        // of the low parts dropped); the mixed terms in FP16 (four factors rounded to 2^-11 of at most
-        // M); r' = r (1 + sigma) in FP32 also in the phase of the wave's centre
+        // of the low parts dropped); the mixed terms in FP16 (four factors rounded to 2^-11), of at most M,
+        // or with the sum along mu split as well of the part across mu and of the second order (with one
+        // more factor)
         const double trunc = sep_trunc(h, v, rho);
         if (!(trunc <= kSepTruncRev)) return std::numeric_limits<double>::infinity();
-        const double M = kTwoPi * h->sep_mixed_max[sep_shape(v)] * rho * (1.0 + sig);
-        e += kSinCosErrRev + 4.0 * u24 * B + trunc + (M * 0x1p-9 + 12.0 * u24) * kInv2Pi;
+        const double r = kTwoPi * rho * (1.0 + sig);
+        const double M = h->sep_mixed_max[sep_shape(v)] * r;
+        const double M16 = v == kTileSep16Q ? h->sep_rest_max[sep_shape(v)] * r + M * (0.625 * M + 0x1p-11) : M;
+        e += kSinCosErrRev + trunc + (M16 * 0x1p-9 + 12.0 * u24) * kInv2Pi;
         return e;
     }
     if (tile_pair(v)) {

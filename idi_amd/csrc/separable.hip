@@ -16,7 +16,7 @@
 // The sums without a remainder keep FP32's precision: X and Y are formed in FP32 and split into two
 // FP16 parts each (22 bits; X_hi Y_hi + X_hi Y_lo + X_lo Y_hi, the products exact, the sums in FP32).
 // The split by itself costs 7e-8 relative L2.  The remainder's sums are weighted by M and need 1e-3
-// of that: the high parts alone.  The image of 100000 emitters on 512 x 512 pixels is within 6.9e-7
+// of that: the high parts alone (variant 22, whose M is ten times as large, splits the one along mu).  The image of 100000 emitters on 512 x 512 pixels is within 6.9e-7
 // of 64 bits (7.5e-7 with the mirror pairs of variant 13), 12345 emitters on 333 x 211 in the far
 // field within 4.6e-7 (6.2e-7).
 //
@@ -95,14 +95,16 @@ __device__ __forceinline__ half2_t rot90(half2_t v)
 }
 
 // Shape of a kernel.  T: rows of a wave's rectangle and columns of its NB blocks (T x NB T pixels);
-// NE: directions along which the mixed remainder is kept (3: all; 2: sep_basis_of); Q2: the
-// second-order term.
+// NE: directions along which the mixed remainder is kept (3: all; 2: sep_basis_of); Q2: for larger
+// remainders (M of 1e-2), the second-order term along mu, and the first-order sum along mu with both
+// parts of the split, as FP16's rounding of M would come near the tolerance.
 template <int T_, int NB_, int NE_, bool Q2_>
 struct SepShape {
     static constexpr int T = T_, NB = NB_, NE = NE_;
     static constexpr bool Q2 = Q2_;
     static constexpr int R = SepTraits<T>::kRegs, kStep = SepTraits<T>::kStep;
     static constexpr int kRows = 2 * T, kCols = 2 * T * NB;  // workgroup tile: 2 x 2 waves
+    static constexpr bool kBasis = NE == 2 || Q2;  // the remainder along the wave's own directions
     static constexpr bool kLdsSums = T == 32;  // compensated sums in LDS (registers hold only T = 16's)
     static constexpr int kStoreUnroll = kLdsSums ? 1 : NB * R;  // the FP64 store is long
     // emitters staged at a time: two per lane where one workgroup fills a CU, so that the FP64 chains of
@@ -124,15 +126,15 @@ struct SepAcc {
 template <class S>
 struct SepLds {
     float4 r[S::kSlots];  // r' (scaled), A
-    // the weights of the remainder's sums as FP16: r' (NE = 3, as (x, y) and
-    // (z, z); the same for all waves), or its
-    // components along the two directions of each wave's rectangle (NE = 2)
-    half2_t h[S::NE == 2 ? 4 : 2][S::kSlots];
+    // the weights of the remainder's sums as FP16: r' as (x, y) and (z, z), the same for all waves, or its
+    // components along the directions of each wave's rectangle: both (NE = 2), or the two across mu (Q2)
+    half2_t h[S::kBasis ? 4 : 2][S::kSlots];
     float amp[S::kSlots];
-    half2_t c2[S::Q2 ? 4 : 1][S::Q2 ? S::kSlots : 1];  // (mu' . r')^2 of each wave, twice
+    float c[S::Q2 ? 4 : 1][S::Q2 ? S::kSlots : 1];     // mu' . r' of each wave
+    half2_t c2[S::Q2 ? 4 : 1][S::Q2 ? S::kSlots : 1];  // its square, twice
     float k[S::kLdsSums ? 4 : 1][S::kLdsSums ? 4 * S::NB * S::R : 1][64];
     float amax[4];
-    float b[4][2][3];
+    float b[4][3][3];  // orthonormal directions of each wave's rectangle, mu / |mu| first
 };
 
 // The operands of one step of kStep emitters: X (high and low parts), its products with the
@@ -141,6 +143,7 @@ struct SepLds {
 template <class S>
 struct SepFrags {
     Frag xh, xl, x1[S::NE], x2;
+    Frag ch, cl;  // Q2: X mu' . r'
     Frag yh[S::NB], yl[S::NB], zh[S::NB], zl[S::NB];
 };
 
@@ -149,7 +152,7 @@ template <class S>
 struct SepRecs {
     float4 r[4];
     half2_t h[4], z[4], c2[4];
-    float a[4];
+    float a[4], c[4];
 };
 
 // e: the lane's first of four emitters.  AMP: the phasors carry the amplitudes.
@@ -159,9 +162,12 @@ __device__ __forceinline__ void sep_load(const SepLds<S>& s, int e, int w, SepRe
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         q.r[i] = s.r[e + i];
-        q.h[i] = s.h[S::NE == 2 ? w : 0][e + i];
-        if constexpr (S::NE == 3) q.z[i] = s.h[1][e + i];
-        if constexpr (S::Q2) q.c2[i] = s.c2[w][e + i];
+        q.h[i] = s.h[S::kBasis ? w : 0][e + i];
+        if constexpr (!S::kBasis) q.z[i] = s.h[1][e + i];
+        if constexpr (S::Q2) {
+            q.c[i] = s.c[w][e + i];
+            q.c2[i] = s.c2[w][e + i];
+        }
         if (AMP) q.a[i] = s.amp[e + i];
     }
 }
@@ -183,10 +189,14 @@ __device__ __forceinline__ void sep_gen(const SepRecs<S>& q, const float (&gx)[3
             sn *= q.a[i];
         }
         split_half(c, sn, f.xh.p[i], f.xl.p[i]);
-        f.x1[0].p[i] = f.xh.p[i] * half2_t{h0.x, h0.x};
-        f.x1[1].p[i] = f.xh.p[i] * half2_t{h0.y, h0.y};
-        if constexpr (S::NE == 3) f.x1[2].p[i] = f.xh.p[i] * q.z[i];
-        if constexpr (S::Q2) f.x2.p[i] = f.xh.p[i] * q.c2[i];
+        constexpr int k0 = S::Q2 ? 1 : 0;
+        f.x1[k0].p[i] = f.xh.p[i] * half2_t{h0.x, h0.x};
+        f.x1[k0 + 1].p[i] = f.xh.p[i] * half2_t{h0.y, h0.y};
+        if constexpr (!S::kBasis) f.x1[2].p[i] = f.xh.p[i] * q.z[i];
+        if constexpr (S::Q2) {
+            f.x2.p[i] = f.xh.p[i] * q.c2[i];
+            split_half(c * q.c[i], sn * q.c[i], f.ch.p[i], f.cl.p[i]);
+        }
 #pragma unroll
         for (int b = 0; b < S::NB; ++b) {
             float u = gy[b][0] * r.x;
@@ -209,8 +219,8 @@ __device__ __forceinline__ void sep_mma(const SepFrags<S>& f, SepAcc<S>& acc)
         Tr::mma(f.xh, f.zh[b], acc.e0[b][1]);
 #pragma unroll
         for (int k = 0; k < S::NE; ++k) {
-            Tr::mma(f.x1[k], f.yh[b], acc.e1[b][k][0]);
-            Tr::mma(f.x1[k], f.zh[b], acc.e1[b][k][1]);
+            Tr::mma(S::Q2 && k == 0 ? f.ch : f.x1[k], f.yh[b], acc.e1[b][k][0]);
+            Tr::mma(S::Q2 && k == 0 ? f.ch : f.x1[k], f.zh[b], acc.e1[b][k][1]);
             if (k == 0) {
                 Tr::mma(f.xh, f.yl[b], acc.e0[b][0]);
                 Tr::mma(f.xh, f.zl[b], acc.e0[b][1]);
@@ -219,6 +229,10 @@ __device__ __forceinline__ void sep_mma(const SepFrags<S>& f, SepAcc<S>& acc)
         if constexpr (S::Q2) {
             Tr::mma(f.x2, f.yh[b], acc.e2[b][0]);
             Tr::mma(f.x2, f.zh[b], acc.e2[b][1]);
+            Tr::mma(f.ch, f.yl[b], acc.e1[b][0][0]);
+            Tr::mma(f.ch, f.zl[b], acc.e1[b][0][1]);
+            Tr::mma(f.cl, f.yh[b], acc.e1[b][0][0]);
+            Tr::mma(f.cl, f.zh[b], acc.e1[b][0][1]);
         }
         Tr::mma(f.xl, f.yh[b], acc.e0[b][0]);
         Tr::mma(f.xl, f.zh[b], acc.e0[b][1]);
@@ -231,8 +245,8 @@ __device__ __forceinline__ void sep_mma(const SepFrags<S>& f, SepAcc<S>& acc)
 template <class S>
 __device__ __forceinline__ void sep_interleave()
 {
-    constexpr int kMma = S::NB * (6 + 2 * S::NE + (S::Q2 ? 2 : 0));
-    constexpr int kValu = 4 * (8 + S::NE + (S::Q2 ? 1 : 0) + 10 * S::NB);
+    constexpr int kMma = S::NB * (6 + 2 * S::NE);  // not used with Q2
+    constexpr int kValu = 4 * (8 + S::NE + 10 * S::NB);
 #pragma unroll
     for (int i = 0; i < kMma; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -294,7 +308,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
             for (int k = 0; k < 3; ++k) gy[b][k] = (float)(-g.krev * (fy.u[k] - fc.u[k])) * inv;
         }
     }
-    if ((Q2 || NE == 2) && l == 0) {
+    if (S::kBasis && l == 0) {
         double r[3];
         pixel_pos(g, sx + (double)hx, sy + (double)hy, r);
         float b[2][3];
@@ -303,6 +317,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
         for (int k = 0; k < 3; ++k) {
             s.b[w][0][k] = b[0][k];
             s.b[w][1][k] = b[1][k];
+            s.b[w][2][k] = b[0][(k + 1) % 3] * b[1][(k + 2) % 3] - b[0][(k + 2) % 3] * b[1][(k + 1) % 3];
         }
     }
 
@@ -364,23 +379,24 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
                 }
                 const float x = r.x * g.sepscale, y = r.y * g.sepscale, z = r.z * g.sepscale;
                 s.r[j] = make_float4(x, y, z, r.A);
-                if constexpr (NE == 2) {
+                if constexpr (S::kBasis) {
+                    constexpr int k0 = Q2 ? 1 : 0;
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        s.h[v][j] = half2_t{(_Float16)(s.b[v][0][0] * x + s.b[v][0][1] * y + s.b[v][0][2] * z),
-                                            (_Float16)(s.b[v][1][0] * x + s.b[v][1][1] * y + s.b[v][1][2] * z)};
+                    for (int v = 0; v < 4; ++v) {
+                        const float(*d)[3] = s.b[v];
+                        s.h[v][j] = half2_t{(_Float16)(d[k0][0] * x + d[k0][1] * y + d[k0][2] * z),
+                                            (_Float16)(d[k0 + 1][0] * x + d[k0 + 1][1] * y + d[k0 + 1][2] * z)};
+                        if constexpr (Q2) {
+                            const float q = d[0][0] * x + d[0][1] * y + d[0][2] * z;
+                            s.c[v][j] = q;
+                            s.c2[v][j] = half2_t{(_Float16)(q * q), (_Float16)(q * q)};
+                        }
+                    }
                 } else {
                     s.h[0][j] = half2_t{(_Float16)x, (_Float16)y};
                     s.h[1][j] = half2_t{(_Float16)z, (_Float16)z};
                 }
                 if (HAS_AMP) s.amp[j] = r.amp * ascale;
-                if constexpr (Q2) {
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const float q2 = s.b[v][0][0] * x + s.b[v][0][1] * y + s.b[v][0][2] * z;
-                        s.c2[v][j] = half2_t{(_Float16)(q2 * q2), (_Float16)(q2 * q2)};
-                    }
-                }
             }
             if (!HAS_AMP) npad = (float)((pad - cnt) & 1);
             __syncthreads();
@@ -445,7 +461,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
 #pragma unroll
             for (int k = 0; k < NE; ++k) {
                 float mk = m[k];
-                if constexpr (NE == 2) mk = m[0] * s.b[w][k][0] + m[1] * s.b[w][k][1] + m[2] * s.b[w][k][2];
+                if constexpr (S::kBasis) mk = m[0] * s.b[w][k][0] + m[1] * s.b[w][k][1] + m[2] * s.b[w][k][2];
                 ar = fmaf(mk, acc.e1[b][k][0][i], ar);
                 ai = fmaf(mk, acc.e1[b][k][1][i], ai);
             }
@@ -497,6 +513,44 @@ __global__ __launch_bounds__(kBlock, S::kWaves) void k_fwd_sep(Geom g, const dou
     }
 }
 
+// Persistent batched form (the queue protocol of k_batched_split).
+template <class S, bool HAS_AMP>
+__global__ __launch_bounds__(kBlock, S::kWaves) void k_batched_sep(Geom g0, const double* __restrict__ emit,
+                                                                   const double* __restrict__ amp,
+                                                                   const WorkItem* __restrict__ items, int nitems,
+                                                                   int* __restrict__ counter, int tiles_y, void* out,
+                                                                   int kind)
+{
+    __shared__ SepLds<S> s;
+    __shared__ int s_item;
+    const size_t npix = (size_t)g0.n0 * g0.n1;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) s_item = atomicAdd(counter, 1);
+        __syncthreads();
+        const int it = s_item;
+        if (it >= nitems) break;
+        const WorkItem wi = items[it];
+        const Geom g = item_geom();
+        const int tx0 = (wi.tile / tiles_y) * S::kRows, ty0 = (wi.tile % tiles_y) * S::kCols;
+        SepOut<S> o;
+        sep_tile<S, HAS_AMP>(g, emit, amp, wi.e0, wi.e1, tx0, ty0, s, o);
+        char* outs = static_cast<char*>(out) +
+                     (size_t)wi.shot * npix * (kind == OUT_INTENSITY ? sizeof(float) : sizeof(float2));
+        const Geom gs = item_geom();  // as in k_batched_pair
+#pragma unroll S::kStoreUnroll
+        for (int i = 0; i < S::NB * S::R; ++i) {
+            int x, y;
+            sep_pixel<S>(tx0, ty0, threadIdx.x >> 6, threadIdx.x & 63, i, x, y);
+            if (x < gs.n0 && y < gs.n1)
+                store_split(gs, x, y, (double)o.at(0, i) - (double)o.at(2, i), (double)o.at(1, i) - (double)o.at(3, i),
+                            outs, kind, (size_t)x * gs.n1 + y);
+        }
+    }
+}
+
+__global__ void k_sep_reset(int* counter) { *counter = 0; }
+
 template <class S, bool A>
 static hipError_t launch_sep_t(const Geom& g, const double* emit, const double* amp, int64_t n, int splits,
                                float4* partial, void* out, int kind, hipStream_t st)
@@ -505,6 +559,24 @@ static hipError_t launch_sep_t(const Geom& g, const double* emit, const double* 
     hipLaunchKernelGGL((k_fwd_sep<S, A>), dim3(tiles_x * tiles_y, splits), dim3(kBlock), 0, st, g, emit, amp, n,
                        tiles_y, split_size(n, splits), partial, out, kind);
     return hipGetLastError();
+}
+
+template <class S, bool A>
+static hipError_t launch_batched_sep_t(const Geom& g, const double* emit, const double* amp, const WorkItem* items,
+                                       int nitems, int* counter, int nblocks, void* out, int kind, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_sep_reset, dim3(1), dim3(1), 0, st, counter);
+    hipLaunchKernelGGL((k_batched_sep<S, A>), dim3(nblocks), dim3(kBlock), 0, st, g, emit, amp, items, nitems, counter,
+                       (g.n1 + S::kCols - 1) / S::kCols, out, kind);
+    return hipGetLastError();
+}
+
+template <class S, bool A>
+static int occupancy_sep_t()
+{
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_batched_sep<S, A>, kBlock, 0) != hipSuccess) return 1;
+    return nb > 0 ? nb : 1;
 }
 
 using Sep32 = SepShape<32, 1, 2, false>;
@@ -531,6 +603,21 @@ hipError_t launch_fwd_sep(int v, bool a, const Geom& g, const double* emit, cons
     if (!(g.sepscale > 0.f) || (g.foldw == 0 && (g.nf || g.secondorder))) return hipErrorInvalidValue;
     IDISIM_DISPATCH_SEP(launch_sep_t, g, emit, amp, n, splits, partial, out, kind, st)
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_batched_sep(int v, bool a, const Geom& g, const double* emit, const double* amp,
+                              const WorkItem* items, int nitems, int* counter, int nblocks, void* out, int kind,
+                              hipStream_t st)
+{
+    if (!(g.sepscale > 0.f) || (g.foldw == 0 && (g.nf || g.secondorder))) return hipErrorInvalidValue;
+    IDISIM_DISPATCH_SEP(launch_batched_sep_t, g, emit, amp, items, nitems, counter, nblocks, out, kind, st)
+    return hipErrorInvalidValue;
+}
+
+int occupancy_batched_sep(int v, bool a)
+{
+    IDISIM_DISPATCH_SEP(occupancy_sep_t)
+    return 1;
 }
 
 }  // namespace idisim

@@ -76,6 +76,37 @@ def test_phase_models(lib, oracle_mod, tile, mode):
     assert rel_l2(I, np.abs(ref) ** 2) <= 1e-4
 
 
+@pytest.mark.parametrize("tile", TILES)
+def test_batched_equals_single_shot(lib, oracle_mod, tile):
+    """The persistent kernel against the single-shot one of the same tile without a split, bit for bit:
+    uneven shots, one empty, a detector that ends inside a tile."""
+    import torch
+
+    from oracle import Geometry
+
+    rng = np.random.default_rng(53)
+    g = Geometry(70, 135, 50.0, 5e5, K_UM, nf=True)
+    sizes = [700, 0, 1, 1500, 513]
+    shots = [atoms_ball(rng, n, 0.01) for n in sizes]
+    amps = [rng.uniform(0.5, 1.0, n) for n in sizes]
+    offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
+    hb, hs = make_handle(lib, g, 1), make_handle(lib, g, 1)
+    for h in (hb, hs):
+        h.set_option(lib.OPT_TILE, tile)
+        h.set_option(lib.OPT_SPLIT, 1)
+    cat, acat = torch.from_numpy(np.concatenate(shots)).cuda(), torch.from_numpy(np.concatenate(amps)).cuda()
+    for amp in (None, acat):
+        out = hb.forward_batched(cat, offsets, amp, extent=0.01).cpu().numpy()
+        assert hb.plan()["tile"] == tile and hb.plan()["phase_bound"] <= 5e-6
+        for s, at in enumerate(shots):
+            if sizes[s] == 0:
+                assert np.count_nonzero(out[s]) == 0
+                continue
+            a = None if amp is None else torch.from_numpy(amps[s]).cuda()
+            single = hs.forward(torch.from_numpy(at).cuda(), a, extent=0.01).cpu().numpy()
+            np.testing.assert_array_equal(out[s], single)
+
+
 def test_rule(lib, oracle_mod):
     """From 5e8 pairs on a field (an intensity from 1e8) takes a separable tile where one meets the bound,
     below it stays on the others; the loss-and-gradient call never does; a geometry whose remainder is too large keeps the
