@@ -21,7 +21,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libidisim.so")
-SOURCES = ["kernels.hip", "separable.hip", "adjoint.hip", "generate.hip", "photons.hip", "correlate.hip", "timesim.hip", "choice.hip", "issue.hip", "idisim.hip"]
+SOURCES = ["kernels.hip", "separable.hip", "adjoint.hip", "adjoint_sep.hip", "generate.hip", "photons.hip", "correlate.hip", "timesim.hip", "choice.hip", "issue.hip", "idisim.hip"]
 ARCH = "gfx950"
 FILE_FLAGS = {}
 

@@ -33,14 +33,13 @@
 //                 FP64 sums are reduced through LDS and written as partials [splits][n][5].
 //   k_adjoint_finalize  sums the partials over splits in FP64.
 // Four emitters per lane measured faster than two or eight at 4096 emitters on 256^2 pixels.
-#include "device_util.hpp"
+#include "adjoint.hpp"
 
 namespace idisim {
 
 namespace {
 constexpr int kAdjWaves = kBlock / 64;  // waves per workgroup
 constexpr int kAdjEPL = 4;              // emitters per lane
-constexpr int kAdjTile = 256;           // pixels per 16 x 16 tile
 
 __device__ inline Frame adj_tile_centre(const Geom& g, int t, int tiles_y)
 {
@@ -51,9 +50,7 @@ __device__ inline Frame adj_tile_centre(const Geom& g, int t, int tiles_y)
 }  // namespace
 
 // The pixel-table entries of pixel (x, y) of 16 x 16 tile t, from its complex64 field value E,
-// its frame f and (nf) its pixel_phasor (cs, sn).
-// target == nullptr: G_p = dLdI[p].  Otherwise the squared-intensity loss L = sum_p (I_p - T_p)^2:
-// G_p = 2 (I_p - T_p) with I_p = |E_p|^2 in FP64, and res2 = (I_p - T_p)^2.
+// its frame f and (nf) its pixel_phasor (cs, sn); res2 as in adj_pixel_weight.
 __device__ inline void adj_pixel_terms(const Geom& g, int t, int tiles_y, int x, int y, const Frame& f, double cs,
                                        double sn, float2 E, const float* __restrict__ dLdI,
                                        const float* __restrict__ target, float4& a, float4& b, float2& c2,
@@ -62,25 +59,8 @@ __device__ inline void adj_pixel_terms(const Geom& g, int t, int tiles_y, int x,
     const Frame c = adj_tile_centre(g, t, tiles_y);
     const double dqx = -g.krev * (f.u[0] - c.u[0]), dqy = -g.krev * (f.u[1] - c.u[1]);
     const double dqz = -g.krev * (f.u[2] - c.u[2]), lam = c.R / f.R;
-    const size_t idx = (size_t)x * g.n1 + y;
-    double G;
-    if (target != nullptr) {
-        const double res = (double)E.x * (double)E.x + (double)E.y * (double)E.y - (double)target[idx];
-        res2 = res * res;
-        G = 2.0 * res;
-    } else {
-        G = (double)dLdI[idx];
-    }
-    double wr = G * (double)E.x, wi = -G * (double)E.y;
-    if (g.nf) {
-        const double r2 = wr * cs - wi * sn;
-        wi = wr * sn + wi * cs;
-        wr = r2;
-    }
-    if (g.scale) {  // the per-pixel factor 1/R_p of the "scale" amplitude R_c/(D_cj R_p)
-        wr /= f.R;
-        wi /= f.R;
-    }
+    double wr, wi;
+    adj_pixel_weight(g, f, cs, sn, E, (size_t)x * g.n1 + y, dLdI, target, wr, wi, res2);
     const double m = sqrt(wr * wr + wi * wi);
     const double psi = (m > 0.0) ? atan2(wi, wr) * kInv2Pi : 0.0;
     a = make_float4((float)dqx, (float)dqy, (float)dqz, (float)psi);
@@ -387,6 +367,14 @@ __global__ __launch_bounds__(256) void k_adjoint_finalize(const double* __restri
     }
 }
 
+hipError_t launch_adjoint_finalize(const double* partial, int splits, int64_t n, float* grad_pos, float* grad_phase,
+                                   float* grad_amp, const double* loss_tile, int ntiles, double* loss, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_adjoint_finalize, dim3((unsigned)((5 * n + 63) / 64)), dim3(256), 0, st, partial, splits, n,
+                       grad_pos, grad_phase, grad_amp, loss_tile, ntiles, loss);
+    return hipGetLastError();
+}
+
 int adjoint_occupancy(bool w, bool lam, bool amp)
 {
     static int cache[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -473,9 +461,8 @@ hipError_t launch_adjoint(bool w, bool lam, const Geom& g, const AdjointLayout& 
         if (a) IDISIM_ADJ_LAUNCH(true, true, true);
         else IDISIM_ADJ_LAUNCH(true, true, false);
     }
-    hipLaunchKernelGGL(k_adjoint_finalize, dim3((unsigned)((5 * n + 63) / 64)), dim3(256), 0, st, partial, L.splits,
-                       n, grad_pos, grad_phase, grad_amp, loss_tile, L.ntiles, target != nullptr ? loss : nullptr);
-    return hipGetLastError();
+    return launch_adjoint_finalize(partial, L.splits, n, grad_pos, grad_phase, grad_amp, loss_tile, L.ntiles,
+                                   target != nullptr ? loss : nullptr, st);
 }
 
 #undef IDISIM_ADJ_LAUNCH

@@ -251,11 +251,21 @@ __host__ __device__ inline SepFrame make_sep_frame(const Geom& g, const double r
     return f;
 }
 
+// The third-order terms of m over -krev, v[0] dx^2 dy + v[1] dx dy^2 (at kappa = 0).
+__host__ __device__ inline void sep_third(const SepFrame& f, double (&v)[2][3])
+{
+    const double pa = f.pa, pb = f.pb, aa = f.aa, bb = f.bb;
+    for (int i = 0; i < 3; ++i) {
+        v[0][i] = (1.5 * aa * pb - 7.5 * pa * pa * pb) * f.p[i] + 3.0 * pa * pb * f.a[i] +
+                  (1.5 * pa * pa - 0.5 * aa) * f.b[i];
+        v[1][i] = (1.5 * bb * pa - 7.5 * pb * pb * pa) * f.p[i] + 3.0 * pa * pb * f.b[i] +
+                  (1.5 * pb * pb - 0.5 * bb) * f.a[i];
+    }
+}
+
 // Two orthonormal directions that hold nearly all of a square's mixed remainder: mu / |mu|, and
-// across it the main direction of the third-order terms
-//   dx^2 dy: -krev / R (...) along -b and p,   dx dy^2: along -a and p,
-// of which the parts across mu span a plane; the larger of the two eigenvectors of their sum of
-// squares.
+// across it the main direction of the third-order terms (the parts of v[0] and v[1] across mu span a
+// plane; the larger of the two eigenvectors of their sum of squares).
 __host__ __device__ inline void sep_basis_of(const SepFrame& f, float (&b)[2][3])
 {
     double e[3] = {f.mu[0], f.mu[1], f.mu[2]};
@@ -263,14 +273,10 @@ __host__ __device__ inline void sep_basis_of(const SepFrame& f, float (&b)[2][3]
     const double n = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
     for (int i = 0; i < 3; ++i) e[i] *= n;
     if (!(n2 > 0.0)) e[0] = 1.0;
-    // coefficients of dx^2 dy and dx dy^2 in m (over a common factor, at kappa = 0)
-    const double pa = f.pa, pb = f.pb, aa = f.aa, bb = f.bb, inv = 1.0 / (aa + bb + pa * pa + pb * pb);
     double v[2][3];
+    sep_third(f, v);
+    const double inv = 1.0 / ((double)f.aa + f.bb + (double)f.pa * f.pa + (double)f.pb * f.pb);
     for (int i = 0; i < 3; ++i) {
-        v[0][i] = (1.5 * aa * pb - 7.5 * pa * pa * pb) * f.p[i] + 3.0 * pa * pb * f.a[i] +
-                  (1.5 * pa * pa - 0.5 * aa) * f.b[i];
-        v[1][i] = (1.5 * bb * pa - 7.5 * pb * pb * pa) * f.p[i] + 3.0 * pa * pb * f.b[i] +
-                  (1.5 * pb * pb - 0.5 * bb) * f.a[i];
         v[0][i] *= inv;
         v[1][i] *= inv;
     }

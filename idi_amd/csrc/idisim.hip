@@ -1298,28 +1298,51 @@ static int adjoint_call(const char* who, idisim_handle* h, const double* emitter
     bool w = false;
     const Geom gl = split_geom(h, adj_tile, &w);
     const bool lam = w && !gl.nf;
-    const AdjointLayout L = adjoint_layout(h->g, n, h->num_cus, adjoint_occupancy(w, lam, grad_amp != nullptr));
+    // The separable form wherever its squares meet the bound: faster from the smallest sizes on (a
+    // call at 16^2 x 1 34 -> 24 us; the kernel at 256^2 x 4096 68 -> 42 us, at 512^2 x 20000 1880 -> 470).  Squares of 32 pixels take 0.6 of the time per
+    // pair of those of 16, where their workgroups fill the device.
+    const bool want_amp = grad_amp != nullptr;
+    bool ws = false;
+    const Geom gs = split_geom(h, kTileSep32V, &ws);
+    int side = gs.foldw || !(gs.nf || gs.secondorder) ? adjoint_sep_side(h, rho) : 0;
+    AdjointSepLayout S{};
+    if (side != 0) {
+        S = adjoint_sep_layout(h->g, side, n, h->num_cus, adjoint_sep_occupancy(side, want_amp));
+        if (side == 32 && S.egroups * S.nwt < 4LL * h->num_cus &&
+            adjoint_sep_bound(h, kTileSep16Q, rho) <= h->tol_rev) {
+            side = 16;
+            S = adjoint_sep_layout(h->g, side, n, h->num_cus, adjoint_sep_occupancy(side, want_amp));
+        }
+    }
+    AdjointLayout L{};
+    if (side == 0) L = adjoint_layout(h->g, n, h->num_cus, adjoint_occupancy(w, lam, want_amp));
+    const size_t bytes = side ? S.bytes : L.bytes;
     float4* fpart = nullptr;
     if (fz != nullptr) {
         // the forward's partials after the adjoint's scratch
-        const size_t off = (L.bytes + 255) / 256 * 256;
+        const size_t off = (bytes + 255) / 256 * 256;
         const size_t fbytes = (size_t)fz->ch.split * h->g.n0 * h->g.n1 * sizeof(float4);
         if (int rc = ensure_scratch(h, off + fbytes)) return rc;
         fpart = reinterpret_cast<float4*>(static_cast<char*>(h->scratch) + off);
         if (int rc = run_forward_partials(h, fz->c, fz->ch.tile, fz->ch.split, fpart)) return rc;
-    } else if (int rc = ensure_scratch(h, L.bytes)) {
+    } else if (int rc = ensure_scratch(h, bytes)) {
         return rc;
     }
-    IDISIM_HIP(launch_adjoint(w, lam, gl, L, emitters, amplitudes, n, static_cast<const float2*>(field), dLdI,
-                              target, loss, h->scratch, grad_pos, grad_phase, grad_amp, st, fpart,
-                              fz ? fz->ch.split : 0, fz ? static_cast<float2*>(const_cast<void*>(field)) : nullptr));
-    const int splits = L.splits;
+    const int fsplit = fz ? fz->ch.split : 0;
+    float2* fout = fz ? static_cast<float2*>(const_cast<void*>(field)) : nullptr;
+    if (side)
+        IDISIM_HIP(launch_adjoint_sep(gs, S, emitters, amplitudes, n, static_cast<const float2*>(field), dLdI, target,
+                                      loss, h->scratch, grad_pos, grad_phase, grad_amp, st, fpart, fsplit, fout));
+    else
+        IDISIM_HIP(launch_adjoint(w, lam, gl, L, emitters, amplitudes, n, static_cast<const float2*>(field), dLdI,
+                                  target, loss, h->scratch, grad_pos, grad_phase, grad_amp, st, fpart, fsplit, fout));
+    const int ran = side == 32 ? kTileSep32V : (side == 16 ? kTileSep16Q : adj_tile);
     h->plan.precision = IDISIM_PREC_FP32SPLIT;
-    h->plan.tile = adj_tile;
-    h->plan.tile_rows = tile_rows(adj_tile);
-    h->plan.tile_cols = tile_cols(adj_tile);
-    h->plan.split = splits;
-    h->plan.phase_bound = bound;
+    h->plan.tile = ran;
+    h->plan.tile_rows = tile_rows(ran);
+    h->plan.tile_cols = tile_cols(ran);
+    h->plan.split = side ? S.splits : L.splits;
+    h->plan.phase_bound = side ? adjoint_sep_bound(h, ran, rho) : bound;
     h->plan.fallback = 0;
     h->plan.graph = 0;
     return IDISIM_OK;

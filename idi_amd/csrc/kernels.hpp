@@ -108,6 +108,24 @@ hipError_t launch_adjoint(bool w, bool lam, const Geom& g, const AdjointLayout& 
                           hipStream_t st, const float4* fwd_partial = nullptr, int fwd_splits = 0,
                           float2* field_out = nullptr);
 
+hipError_t launch_adjoint_finalize(const double* partial, int splits, int64_t n, float* grad_pos, float* grad_phase,
+                                   float* grad_amp, const double* loss_tile, int ntiles, double* loss, hipStream_t st);
+
+// The separable adjoint (adjoint_sep.hip) over T x T pixel squares (T = 16 or 32), W folded.  Its
+// scratch: the squares' tables, the split partials, the tiles' loss parts.
+struct AdjointSepLayout {
+    int T, sq_x, sq_y, wt_y, nwt, per, splits, ntiles;  // squares, workgroup tiles (2 x 2), per workgroup; 16 x 16 tiles
+    int64_t egroups;
+    size_t tab_bytes, part_bytes, bytes;
+};
+AdjointSepLayout adjoint_sep_layout(const Geom& g, int T, int64_t n, int num_cus, int blocks_per_cu);
+int adjoint_sep_occupancy(int T, bool amp);
+// arguments as for launch_adjoint
+hipError_t launch_adjoint_sep(const Geom& g, const AdjointSepLayout& L, const double* emit, const double* amp,
+                              int64_t n, const float2* field, const float* dLdI, const float* target, double* loss,
+                              void* scratch, float* grad_pos, float* grad_phase, float* grad_amp, hipStream_t st,
+                              const float4* fwd_partial = nullptr, int fwd_splits = 0, float2* field_out = nullptr);
+
 hipError_t launch_extent(const double* emit, int64_t n, unsigned long long* out, hipStream_t st);
 // issue-rate probe (kind 0: v_fma_f32, 1: v_sin_f32 / v_cos_f32); out: blocks x 256 floats
 hipError_t launch_issue_probe(int kind, int blocks, int iters, float* out, hipStream_t st);

@@ -39,9 +39,10 @@ struct Planner {
     double cent_coef = 0.0;   // largest |(m_0 - m_1) - (m_0 - m_1) of the sub-block reference| (variant 15)
     double lin_coef = 0.0;    // largest residual of the linear wave reference (variant 13) per unit extent
     // separable tiles, wave rectangles of 32 x 32 (0), 32 x 64 (1) and 16 x 16 (2) pixels: the largest
-    // column phase, the largest mixed remainder |m|, its largest part beyond dx dy mu and beyond
-    // the two directions of sep_basis_of, per unit extent (rev per length)
+    // column phase, the largest mixed remainder |m|, its largest part beyond dx dy mu, beyond
+    // the two directions of sep_basis_of and beyond the third order, per unit extent (rev per length)
     double sep_line_max[3] = {}, sep_mixed_max[3] = {}, sep_rest_max[3] = {}, sep_off_max[3] = {};
+    double sep_fourth_max[3] = {};
 };
 
 // The truncation (revolutions) that a separable tile may leave.  Its relative L2 error is about a
@@ -226,7 +227,7 @@ inline void planner_sep_tables(Planner* h)
     for (int t = 0; t < 3; ++t) {
         const int TX = t == 2 ? 16 : 32, TY = t == 1 ? 64 : TX;
         const double hx = 0.5 * (TX - 1), hy = 0.5 * (TY - 1);
-        double line = 0.0, worst = 0.0, rest = 0.0, off = 0.0, du = 0.0, dR = 0.0;
+        double line = 0.0, worst = 0.0, rest = 0.0, off = 0.0, fourth = 0.0, du = 0.0, dR = 0.0;
         bool ok = (int64_t)g.n0 * g.n1 <= (int64_t)2048 * 2048;
         for (int x0 = 0; x0 < g.n0 && ok; x0 += TX) {
             for (int y0 = 0; y0 < g.n1 && ok; y0 += TY) {
@@ -241,6 +242,8 @@ inline void planner_sep_tables(Planner* h)
                 ok = e < 0.01;
                 float b[2][3];
                 sep_basis_of(sf, b);
+                double v3[2][3];
+                sep_third(sf, v3);
                 const Frame wc = pixel_frame(g, x0 / (2 * TX) * (2 * TX) + TX - 0.5, y0 / (2 * TY) * (2 * TY) + TY - 0.5);
                 const Frame fx[2] = {pixel_frame(g, cx - hx, cy), pixel_frame(g, cx + hx, cy)};
                 const Frame fy[2] = {pixel_frame(g, cx, cy - hy), pixel_frame(g, cx, cy + hy)};
@@ -248,16 +251,18 @@ inline void planner_sep_tables(Planner* h)
                     for (int j = 0; j < 2; ++j) {
                         const Frame f = pixel_frame(g, cx + (2 * i - 1) * hx, cy + (2 * j - 1) * hy);
                         const double dd = (2 * i - 1) * (2 * j - 1) * hx * hy;
-                        double m[3], u2 = 0.0, m2 = 0.0, s2 = 0.0, o2 = 0.0, m0 = 0.0, m1 = 0.0, lx = 0.0, ly = 0.0;
+                        double m[3], u2 = 0.0, m2 = 0.0, s2 = 0.0, o2 = 0.0, f2 = 0.0, m0 = 0.0, m1 = 0.0, ly = 0.0;
+                        const double ex = (2 * i - 1) * hx, ey = (2 * j - 1) * hy;
                         for (int k = 0; k < 3; ++k) {
-                            const double dx = g.krev * (fx[i].u[k] - c.u[k]), dy = g.krev * (fy[j].u[k] - c.u[k]);
+                            const double dy = g.krev * (fy[j].u[k] - c.u[k]);
                             m[k] = -g.krev * ((f.u[k] - fx[i].u[k]) - (fy[j].u[k] - c.u[k]));
                             const double s = m[k] - dd * (double)sf.mu[k];
                             u2 += (f.u[k] - wc.u[k]) * (f.u[k] - wc.u[k]);
-                            lx += dx * dx;
                             ly += dy * dy;
                             m2 += m[k] * m[k];
                             s2 += s * s;
+                            const double q = s + g.krev * ex * ey * (ex * v3[0][k] + ey * v3[1][k]);
+                            f2 += q * q;
                             m0 += m[k] * (double)b[0][k];
                             m1 += m[k] * (double)b[1][k];
                         }
@@ -271,6 +276,7 @@ inline void planner_sep_tables(Planner* h)
                         worst = std::max(worst, std::sqrt(m2));
                         rest = std::max(rest, std::sqrt(s2));
                         off = std::max(off, std::sqrt(o2));
+                        fourth = std::max(fourth, std::sqrt(f2));
                     }
                 }
             }
@@ -279,6 +285,7 @@ inline void planner_sep_tables(Planner* h)
         h->sep_mixed_max[t] = ok ? 1.05 * worst : inf;
         h->sep_rest_max[t] = ok ? 1.05 * rest : inf;
         h->sep_off_max[t] = ok ? 1.05 * off : inf;
+        h->sep_fourth_max[t] = ok ? 1.05 * fourth : inf;
         for (int v = kTileSep32; v < kNumTilesAll; ++v) {
             if (sep_shape(v) != t) continue;
             h->du_max[v] = 1.05 * du;
@@ -349,6 +356,17 @@ inline double sep_trunc(const Planner* h, int v, double rho)
     return (0.5 * M * M + off) * kInv2Pi;
 }
 
+// FP16's rounding of the mixed terms of the separable tile v (revolutions): four factors rounded to
+// 2^-11, of at most M, or, with the sum along mu split (kTileSep16Q), of the part across mu and of the
+// second order (one more factor).
+inline double sep_half_error(const Planner* h, int v, double rho)
+{
+    const double r = kTwoPi * rho * (1.0 + sigma_bound(h, v, rho));
+    const double M = h->sep_mixed_max[sep_shape(v)] * r;
+    const double M16 = v == kTileSep16Q ? h->sep_rest_max[sep_shape(v)] * r + M * (0.625 * M + 0x1p-11) : M;
+    return M16 * 0x1p-9 * kInv2Pi;
+}
+
 // A-priori bound of the per-term phase error (revolutions) of tile variant v
 // for emitters within |r_j| <= rho.
 inline double plan_bound(const Planner* h, int v, double rho)
@@ -399,15 +417,10 @@ inline double plan_bound(const Planner* h, int v, double rho)
     }
     if (tile_sep(v)) {
         // a second sincos; the phasors split into two FP16 parts each (2^-23 per component, the product
-        // of the low parts dropped); the mixed terms in FP16 (four factors rounded to 2^-11), of at most M,
-        // or with the sum along mu split as well of the part across mu and of the second order (with one
-        // more factor)
+        // of the low parts dropped); the mixed terms
         const double trunc = sep_trunc(h, v, rho);
         if (!(trunc <= kSepTruncRev)) return std::numeric_limits<double>::infinity();
-        const double r = kTwoPi * rho * (1.0 + sig);
-        const double M = h->sep_mixed_max[sep_shape(v)] * r;
-        const double M16 = v == kTileSep16Q ? h->sep_rest_max[sep_shape(v)] * r + M * (0.625 * M + 0x1p-11) : M;
-        e += kSinCosErrRev + trunc + (M16 * 0x1p-9 + 12.0 * u24) * kInv2Pi;
+        e += kSinCosErrRev + trunc + sep_half_error(h, v, rho) + 12.0 * u24 * kInv2Pi;
         return e;
     }
     if (tile_pair(v)) {
@@ -447,6 +460,31 @@ inline double plan_bound(const Planner* h, int v, double rho)
         }
     }
     return e;
+}
+
+// The phase bound (revolutions) of the separable adjoint (adjoint_sep.hip) with the squares of tile v
+// (kTileSep32V or kTileSep16Q): that of the forward's phases without its mixed terms, one rounding for
+// the weights, and what the adjoint leaves of m beyond the terms that it keeps: M^2 / 2 (in the sums
+// weighted by dq) and the fourth order.
+inline double adjoint_sep_bound(const Planner* h, int v, double rho)
+{
+    const double inf = std::numeric_limits<double>::infinity();
+    const int t = sep_shape(v);
+    const double r = kTwoPi * rho * (1.0 + sigma_bound(h, v, rho));
+    const double M = h->sep_mixed_max[t] * r;
+    const double trunc = (0.5 * M * M + h->sep_fourth_max[t] * r) * kInv2Pi;
+    const double b = plan_bound(h, v, rho);
+    if (!(trunc <= kSepTruncRev) || !std::isfinite(b)) return inf;
+    return b - sep_trunc(h, v, rho) - sep_half_error(h, v, rho) + trunc + 0x1p-23;
+}
+
+// Side of the squares with which it meets the tolerance for emitters within |r_j| <= rho, 32 or 16, or
+// 0.
+inline int adjoint_sep_side(const Planner* h, double rho)
+{
+    for (int v : {kTileSep32V, kTileSep16Q})
+        if (adjoint_sep_bound(h, v, rho) <= h->tol_rev) return tile_sep_rows(v);
+    return 0;
 }
 
 // Tile variants of the FP32-split kernels whose error bound meets the tolerance.

@@ -31,68 +31,15 @@
 // matrix cores 0.5, and the clock at 1.83 GHz (2.24 under the mirror-pair kernel).  That image takes
 // 1.07 ms against 3.29 ms with variant 13.  Sharing X between two blocks of columns (variants 19, 20:
 // one wave per SIMD, 512 registers) saves a quarter of the VALU and 10 to 14% of the time.
-#include "device_util.hpp"
+#include "mfma_util.hpp"
 
 namespace idisim {
 
 namespace {
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
-
-union Frag {
-    half8_t v;
-    half2_t p[4];
-};
-
 // Emitters between two merges of the FP32 sums into the compensated ones.  An instruction adds the
 // products of 8 or 16 emitters before it rounds into its sum, so 512 emitters see no more roundings
 // than the 256 single additions of the other tiles.
 constexpr int kSepMerge = 512;
-
-template <int T>
-struct SepTraits;
-template <>
-struct SepTraits<32> {
-    using acc_t = float16_t;
-    static constexpr int kStep = 8, kRegs = 16;
-    static __device__ __forceinline__ void mma(const Frag& a, const Frag& b, acc_t& c)
-    {
-        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.v, b.v, c, 0, 0, 0);
-    }
-    // row of accumulator register i in lane group g = lane / 32
-    static __device__ __forceinline__ int row(int i, int g) { return 8 * (i >> 2) + 4 * g + (i & 3); }
-};
-template <>
-struct SepTraits<16> {
-    using acc_t = float4_t;
-    static constexpr int kStep = 16, kRegs = 4;
-    static __device__ __forceinline__ void mma(const Frag& a, const Frag& b, acc_t& c)
-    {
-        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v, b.v, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int i, int g) { return 4 * g + i; }
-};
-
-// (c, s) as FP16 pairs: h rounded to nearest, l the remainder rounded to nearest.
-__device__ __forceinline__ void split_half(float c, float s, half2_t& h, half2_t& l)
-{
-    h = __builtin_convertvector((float2_t{c, s}), half2_t);
-    asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mixhi_f16 %0, -%1, 1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "=&v"(l)
-        : "v"(h), "v"(c), "v"(s));
-}
-
-// (x, y) -> (-y, x)
-__device__ __forceinline__ half2_t rot90(half2_t v)
-{
-    half2_t r;
-    asm("v_pk_mul_f16 %0, %1, 1.0 op_sel:[1,0] op_sel_hi:[0,0] neg_lo:[1,0]" : "=v"(r) : "v"(v));
-    return r;
-}
 
 // Shape of a kernel.  T: rows of a wave's rectangle and columns of its NB blocks (T x NB T pixels);
 // NE: directions along which the mixed remainder is kept (3: all; 2: sep_basis_of); Q2: for larger
