@@ -137,3 +137,29 @@ def test_qcorr_wide_image_unstaged_rows():
     _lib.qcorr(torch.from_numpy(zd).cuda(), torch.from_numpy(img).cuda(), xc, yc, 500.0, qmax, maxdqz, out)
     np.testing.assert_allclose(out.cpu().numpy(), qcorr(zd, img, xc, yc, 500.0, qmax, maxdqz), rtol=1e-12,
                                atol=1e-11)
+
+
+@pytest.mark.parametrize("shape,maxq,z", [((32, 20), 32, 500.0), ((33, 64), 32, 80.0), ((40, 65), 40, 300.0),
+                                          ((129, 191), 48, 150.0), ((70, 130), 64, 4000.0)])
+@pytest.mark.parametrize("smooth", [True, False])
+def test_qcorr_runs_at_the_edges(shape, maxq, z, smooth):
+    """Images narrower than the column offsets, at and past the edges of the column blocks and offset groups,
+    bins beyond the window that a workgroup keeps (a strong curvature; a zd that is noise, so that every
+    pair changes the bin)."""
+    import torch
+
+    from idi_amd import _lib
+    from idi_amd.reconstruction.qcor import geometry
+    from oracle.correlate import qcorr
+
+    rng = np.random.default_rng(70)
+    zd, xc, yc, qmax, maxdqz = geometry(shape, z, maxq, 0.37 * shape[0], 0.61 * shape[1])
+    if not smooth:
+        zd = rng.uniform(0.5, 1.0, shape).astype(np.float32)
+        maxdqz = 21
+    img = rng.normal(1, 2, shape).astype(np.float32)
+    out = torch.empty((2 * maxdqz, 2 * qmax, 2 * qmax), dtype=torch.float64, device="cuda")
+    _lib.qcorr(torch.from_numpy(zd).cuda(), torch.from_numpy(img).cuda(), xc, yc, z, qmax, maxdqz, out)
+    want = qcorr(zd, img, xc, yc, z, qmax, maxdqz)
+    # each pair's product is exact; FP64 sums in another order
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=0, atol=2.0**-52 * np.abs(img).sum() ** 2)
