@@ -16,8 +16,8 @@
 // keys on FP32-split handles (the reference's "mixed" precision, which also takes the sine
 // and cosine of the range-reduced phase in FP32) and float64 on FP64 handles.
 //
-// Up to 20480 emitters (float32 keys; 12288 with float64 keys): k_time_fused, one workgroup
-// of 256 or 512 lanes per pixel, all in registers and LDS.
+// Up to 20480 emitters (float32 keys; 12288 with float64 keys): k_time_fused_phase (float32 keys without
+// 1/r) or k_time_fused, one workgroup of 256 or 512 lanes per pixel, all in registers and LDS.
 // Larger counts, per batch of pixels:
 //   k_time_prepare    one thread per (pixel, emitter): key t, index j, amplitude a (FP64);
 //   segmented radix sort of (t, j) per pixel (rocPRIM, stable);
@@ -47,11 +47,10 @@ namespace {
 // reduced to revolutions in FP64 and its sine and cosine taken in FP32
 // (v_sin_f32 / v_cos_f32, ~1e-7 absolute), as the reference's single path takes
 // __sincosf of a float phase.
-template <bool F32AMP>
-__device__ inline void arrival(const Geom& g, const double r[3], double R, const double* e, double T, double c,
-                               double* t, double* re, double* im)
+__device__ inline void arrival_phase(const Geom& g, const double r[3], double R, const double* e, double T, double c,
+                                     double& t, double& ph, double& scale)
 {
-    double ph, scale = 1.0;
+    scale = 1.0;
     if (g.nf) {
         const double dx = e[0] - r[0], dy = e[1] - r[1], dz = e[2] - r[2];
         const double d = sqrt(dx * dx + dy * dy + dz * dz);
@@ -59,21 +58,35 @@ __device__ inline void arrival(const Geom& g, const double r[3], double R, const
         const double e2 = e[0] * e[0] + e[1] * e[1] + e[2] * e[2];
         const double er = e[0] * r[0] + e[1] * r[1] + e[2] * r[2];
         const double s = (e2 - 2.0 * er) / (d + R) + e[2];
-        *t = s / c + T;
+        t = s / c + T;
         ph = s * g.k + e[3];
         if (g.scale) scale = 1.0 / d;
     } else {
         const double rd = 1.0 / R;
         const double kr = g.k * rd;
         const double s = e[0] * (r[0] * kr) + e[1] * (r[1] * kr) + e[2] * (g.k * (r[2] * rd - 1.0));
-        *t = -s / (c * g.k) + T;
+        t = -s / (c * g.k) + T;
         ph = e[3] - s;
         if (g.scale) scale = rd;
     }
+}
+
+// The phase reduced to revolutions (F32AMP).
+__device__ inline float reduced(double ph)
+{
+    double rv = ph * kInv2Pi;
+    rv -= rint(rv);
+    return (float)rv;
+}
+
+template <bool F32AMP>
+__device__ inline void arrival(const Geom& g, const double r[3], double R, const double* e, double T, double c,
+                               double* t, double* re, double* im)
+{
+    double ph, scale;
+    arrival_phase(g, r, R, e, T, c, *t, ph, scale);
     if (F32AMP) {
-        double rv = ph * kInv2Pi;
-        rv -= rint(rv);
-        const float fr = (float)rv;
+        const float fr = reduced(ph);
         *re = (double)__builtin_amdgcn_cosf(fr) * scale;
         *im = (double)__builtin_amdgcn_sinf(fr) * scale;
     } else {
@@ -369,6 +382,116 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused(Geom g, const double* __re
     if (tid == 0) out[p] = ssum[0] * (0.5 * tau);
 }
 
+// k_time_fused where an amplitude is its phase alone (float32 keys, no 1/r): the FP32 phase goes through
+// the sort with the key, so nothing is computed twice or gathered by emitter, and the sorted arrivals
+// stay in registers.  Equal keys may take any order: the gap between them is 0.
+// One expm1 a gap: with e = expm1(-gap / tau) the decay is 1 + e and the integral's weight -e (2 + e).
+// Bound by the sort (1.5 of 2.5 ms at 128^2 x 10000) and the FP64 arithmetic of arrivals and gaps.
+// k_time_fused -> this: 3370 -> 2500 us there; 256 x 40 arrivals (220 VGPRs, 2 waves a SIMD) 2630,
+// 1024 x 10 3540, 6 bits a pass of the sort 2790, 8 bits 2490.
+template <int ITEMS, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void k_time_fused_phase(Geom g, const double* __restrict__ emit,
+                                                            const double* __restrict__ times, int64_t n, double c,
+                                                            double tau, double* __restrict__ out)
+{
+    using Sort = rocprim::block_radix_sort<float, BLOCK, ITEMS, float>;
+    union Lds {
+        typename Sort::storage_type sort;
+        struct {
+            double re[BLOCK], im[BLOCK], t[BLOCK];
+            int has[BLOCK];
+            float first[BLOCK], last[BLOCK];
+        } scan;
+        double sum[BLOCK];
+    };
+    __shared__ Lds u;
+    const int tid = threadIdx.x;
+    const int64_t p = blockIdx.x;
+    const double inv_tau = 1.0 / tau;
+    double r[3];
+    pixel_pos(g, (double)(p / g.n1), (double)(p % g.n1), r);
+    const double R = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
+
+    float key[ITEMS], ph[ITEMS];
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const int j = tid + k * BLOCK;
+        key[k] = INFINITY;
+        ph[k] = 0.f;
+        if (j < n) {
+            double t, phase, scale;
+            arrival_phase(g, r, R, emit + 4 * (int64_t)j, times[j], c, t, phase, scale);
+            key[k] = (float)t;
+            ph[k] = reduced(phase);
+        }
+    }
+    Sort().sort(key, ph, u.sort);
+    __syncthreads();
+    u.scan.first[tid] = key[0];
+    u.scan.last[tid] = key[ITEMS - 1];
+    __syncthreads();
+    const int i0 = tid * ITEMS;
+    const int cnt = (int)(n - i0 < ITEMS ? (n - i0 > 0 ? n - i0 : 0) : ITEMS);
+    const double tprev = tid > 0 ? (double)u.scan.last[tid - 1] : (double)key[0];
+    const double tnext = tid + 1 < BLOCK ? (double)u.scan.first[tid + 1] : 0.0;
+
+    // the sums A, B, C of k_time_fused
+    double pr = 0.0, pi = 0.0, D = 1.0, tl = tprev, A = 0.0, Br = 0.0, Bi = 0.0, C = 0.0;
+    double d = cnt > 0 ? exp(-((double)key[0] - tprev) * inv_tau) : 1.0;
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        if (k < cnt) {
+            pr = fma(d, pr, (double)__builtin_amdgcn_cosf(ph[k]));
+            pi = fma(d, pi, (double)__builtin_amdgcn_sinf(ph[k]));
+            D *= d;
+            tl = (double)key[k];
+            double w = 1.0;
+            if (i0 + k + 1 < n) {
+                const double tn = k + 1 < ITEMS ? (double)key[k + 1 < ITEMS ? k + 1 : k] : tnext;
+                const double e = expm1((tl - tn) * inv_tau);
+                d = 1.0 + e;
+                w = -e * (2.0 + e);
+            }
+            A = fma(w, pr * pr + pi * pi, A);
+            const double wD = w * D;
+            Br = fma(wD, pr, Br);
+            Bi = fma(wD, pi, Bi);
+            C = fma(wD, D, C);
+        }
+    }
+    const DecayState mine = {pr, pi, tl, cnt > 0 ? 1 : 0};
+    u.scan.re[tid] = mine.re;
+    u.scan.im[tid] = mine.im;
+    u.scan.t[tid] = mine.t;
+    u.scan.has[tid] = mine.has;
+    __syncthreads();
+    DecayState inc = mine;
+    for (int off = 1; off < BLOCK; off <<= 1) {
+        DecayState left = {0.0, 0.0, 0.0, 0};
+        if (tid >= off) left = {u.scan.re[tid - off], u.scan.im[tid - off], u.scan.t[tid - off], u.scan.has[tid - off]};
+        __syncthreads();
+        inc = combine(left, inc, inv_tau);
+        u.scan.re[tid] = inc.re;
+        u.scan.im[tid] = inc.im;
+        u.scan.t[tid] = inc.t;
+        u.scan.has[tid] = inc.has;
+        __syncthreads();
+    }
+    double xr = 0.0, xi = 0.0;
+    if (tid > 0 && u.scan.has[tid - 1]) {
+        xr = u.scan.re[tid - 1];
+        xi = u.scan.im[tid - 1];
+    }
+    __syncthreads();
+    u.sum[tid] = A + 2.0 * (xr * Br + xi * Bi) + (xr * xr + xi * xi) * C;
+    __syncthreads();
+    for (int s2 = BLOCK / 2; s2 > 0; s2 >>= 1) {
+        if (tid < s2) u.sum[tid] += u.sum[tid + s2];
+        __syncthreads();
+    }
+    if (tid == 0) out[p] = u.sum[0] * (0.5 * tau);
+}
+
 template <typename Tt>
 static size_t time_sort_bytes(int np, int64_t n)
 {
@@ -439,6 +562,34 @@ static hipError_t run_fused(const Geom& g, const double* emit, const double* tim
                             double* out, int64_t npix, hipStream_t st)
 {
     const dim3 grid((unsigned)npix);
+    if constexpr (sizeof(Tt) == 4) {
+        if (!g.scale) {
+#define IDISIM_TIME_PHASE(I, B) \
+    hipLaunchKernelGGL((k_time_fused_phase<I, B>), grid, dim3(B), 0, st, g, emit, times, n, c, tau, out)
+            if (n <= 256 * 4)
+                IDISIM_TIME_PHASE(4, 256);
+            else if (n <= 256 * 8)
+                IDISIM_TIME_PHASE(8, 256);
+            else if (n <= 256 * 16)
+                IDISIM_TIME_PHASE(16, 256);
+            else if (n <= 256 * 24)
+                IDISIM_TIME_PHASE(24, 256);
+            else if (n <= 512 * 16)
+                IDISIM_TIME_PHASE(16, 512);
+            else if (n <= 512 * 20)
+                IDISIM_TIME_PHASE(20, 512);
+            else if (n <= 512 * 24)
+                IDISIM_TIME_PHASE(24, 512);
+            else if (n <= 512 * 32)
+                IDISIM_TIME_PHASE(32, 512);
+            else if (n <= 512 * 40)
+                IDISIM_TIME_PHASE(40, 512);
+            else
+                return hipErrorInvalidValue;  // past the fused capacity (time_fused_ok)
+#undef IDISIM_TIME_PHASE
+            return hipGetLastError();
+        }
+    }
 #define IDISIM_TIME_FUSED(I, B) \
     hipLaunchKernelGGL((k_time_fused<Tt, I, B>), grid, dim3(B), 0, st, g, emit, times, n, c, tau, out)
     if (n <= 256 * 4)

@@ -152,3 +152,30 @@ def test_time_paths_agree_across_fused_capacity(lib, n, precision):
         h.set_option(lib.OPT_TIME_PATH, path)
         res.append(h.time_forward(d, t, C_UM_FS, 1e-3).cpu().numpy())
     assert rel_l2(res[0], res[1]) <= 1e-12
+
+
+@pytest.mark.parametrize("n", [255, 256, 1024, 1025, 2049, 4097, 6145, 8192, 8193, 10240, 10241, 12289])
+@pytest.mark.parametrize("nf", [False, True])
+def test_time_phase_kernel_at_its_capacities(lib, nf, n):
+    """The kernels that sort the FP32 phase with the key, at the edges of their sizes, with arrivals that
+    coincide (every emitter twice, equal keys in any order) and a gap of many decay times, against the batched path:
+    FP64 sums of the same terms (the decay as 1 + expm1) in another order; and the same bits again."""
+    import torch
+
+    import oracle
+    from gpu_util import make_handle
+
+    rng = np.random.default_rng(n)
+    at = _atoms(rng, n, 0.02)
+    at[n // 2:2 * (n // 2), :3] = at[:n // 2, :3]
+    times = rng.normal(0, 5e-4, n)
+    times[n // 2:2 * (n // 2)] = times[:n // 2]
+    times[::7] += 0.5
+    times[n // 2:2 * (n // 2)] = times[:n // 2]
+    g = oracle.Geometry(5, 3, 300.0, 1e5, K_UM, nf=nf)
+    h = make_handle(lib, g, lib.PREC_FP32SPLIT)
+    d, t = torch.from_numpy(at).cuda(), torch.from_numpy(times).cuda()
+    a = h.time_forward(d, t, C_UM_FS, 1e-3)
+    assert torch.equal(a, h.time_forward(d, t, C_UM_FS, 1e-3))
+    h.set_option(lib.OPT_TIME_PATH, 2)
+    assert rel_l2(a.cpu().numpy(), h.time_forward(d, t, C_UM_FS, 1e-3).cpu().numpy()) <= 1e-12
