@@ -38,6 +38,12 @@ LAMBDA_UM = 1.54e-4
 K = 2 * np.pi / LAMBDA_UM
 METRIC = "emitter-pixel pair evals/s, 1 GPU: FP32-split vs FP64 at <=1e-4 rel err"
 FP32_PEAK_TFLOPS = 157.3   # MI355X FP32 vector (published, packed)
+FP16_PEAK_TFLOPS = 2500.0  # MI355X FP16 matrix, dense (published)
+FIRST_MATRIX_TILE = 17
+# FP16 matrix flops per emitter-pixel pair: 4 per instruction of a step (10, 12 or 16 of them; the
+# adjoint's 16)
+MATRIX_FLOPS = {17: 40, 18: 48, 19: 40, 20: 48, 21: 40, 22: 64}
+ADJOINT_MATRIX_FLOPS = 64
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 vector (published)
 OPS_PER_PAIR_NF = 23       # near field, unit amplitude: 3 sub, 3 mul + 2 add, sqrt, 4 (phase), cos, sin, 8 (Kahan)
 OPS_PER_PAIR_NF_AMP = 25
@@ -99,6 +105,23 @@ def roofline_valu(lib, mix, pairs_per_s, ops_per_pair, traffic=None, kernel_ms=N
     r["algorithmic"] = {"ops_per_pair": ops_per_pair, "tflops": alg, "frac": alg / FP32_PEAK_TFLOPS}
     r["issue"] = issue_fields(lib, mix, pairs_per_s)
     return r
+
+
+def roofline(lib, family, tile, pairs_per_s, ops_per_pair, amp=False, traffic=None, kernel_ms=None):
+    """Roofline fields of an FP32-split kernel by its tile variant.
+
+    The separable tiles (17 and up) form their sums on the matrix cores: achieved / frac are the FP16
+    matrix flops that the kernel executes (its instructions per step over its pairs per step) against the
+    dense FP16 peak.  The two FP16 parts of each factor and the corrections are in that count, so it says
+    how busy the matrix cores are, not how much work the formula asks for (algorithmic)."""
+    if tile < FIRST_MATRIX_TILE:
+        return roofline_valu(lib, load_mix(family, tile, amp), pairs_per_s, ops_per_pair, traffic, kernel_ms)
+    flops = ADJOINT_MATRIX_FLOPS if family == "adjoint" else MATRIX_FLOPS[tile]
+    achieved, alg = flops * pairs_per_s / 1e12, pairs_per_s * ops_per_pair / 1e12
+    return {"bound": "valu and matrix issue", "achieved": achieved, "peak": FP16_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": achieved / FP16_PEAK_TFLOPS, "matrix_flops_per_pair": flops, "traffic": traffic,
+            "kernel_ms": kernel_ms,
+            "algorithmic": {"ops_per_pair": ops_per_pair, "tflops": alg, "frac": alg / FP32_PEAK_TFLOPS}}
 
 
 def log(*a):
@@ -250,7 +273,7 @@ def bench_single(args):
                          f"({len(rows) * n1 * len(atoms):.3e} pairs, {dt:.1f} s) of the same image; "
                          f"FP64 C/OpenMP restatement of cpu.py:30-107, {cpu_model()}"}
     rate = pairs / (split_ms * 1e-3)
-    roof = roofline_valu(_lib, load_mix("single", plan["tile"]), rate, OPS_PER_PAIR_NF, kernel_ms=split_ms)
+    roof = roofline(_lib, "single", plan["tile"], rate, OPS_PER_PAIR_NF, kernel_ms=split_ms)
     log("roofline", roof)
     traffic = args.traffic
     if traffic is None:
@@ -281,7 +304,8 @@ def bench_single(args):
         "config": {"workload": "near-field image: 100000 of 155331 simple-cubic sites (a=0.3 nm) in a 10 nm ball, "
                                "random phases, 512x512 px of 75 um at z=0.2 m, lambda=0.154 nm",
                    "emitters": len(atoms), "pixels": n0 * n1, "pairs_per_step": pairs,
-                   "precision": "FP32-split (FP64 range-reduced phase, FP32 sincos + chunked Kahan sums)",
+                   "precision": "FP32-split (FP64 range-reduced phase, FP32 sincos + chunked Kahan sums; tiles from 17 on "
+                                "multiply the phasors as two FP16 parts each, 22 bits, into FP32 sums)",
                    "plan": plan},
         "fp64": {"value": value64, "ms_per_step": wall64 * 1e3 / s64, "kernel_ms": float(np.mean(ms64)),
                  "plan": h64.plan()},
@@ -370,8 +394,8 @@ def bench_batched(args):
                        "plan": h.plan()},
             "fp64": f64, "speedup_vs_fp64": (pairs * args.steps / wall) / f64["value"],
             "rel_l2_intensity": {"fp32split_vs_fp64_gpu_all_shots": rel, "fp32split_vs_oracle_rows": rel_oracle},
-            "roofline": roofline_valu(_lib, load_mix("batched", h.plan()["tile"]), pairs / (np.mean(ms) * 1e-3),
-                                      OPS_PER_PAIR_NF, kernel_ms=float(np.mean(ms)))}
+            "roofline": roofline(_lib, "batched", h.plan()["tile"], pairs / (np.mean(ms) * 1e-3),
+                                 OPS_PER_PAIR_NF, kernel_ms=float(np.mean(ms)))}
 
 
 def three_balls(rng, n_total=1_000_000):
@@ -442,8 +466,8 @@ def bench_large(args):
                                    "fresh phases, 16 shots, 1024x1024 px of 50 um at z=0.5 m, near field"
                                    % counts.tolist(), "pairs_per_step": pairs, "plan": h.plan()},
             "rel_l2_intensity": {"fp32split_vs_oracle_rows": rel_oracle},
-            "roofline": roofline_valu(_lib, load_mix("batched", h.plan()["tile"], amp=True),
-                                      pairs / (np.mean(ms) * 1e-3), OPS_PER_PAIR_NF_AMP, kernel_ms=float(np.mean(ms)))}
+            "roofline": roofline(_lib, "batched", h.plan()["tile"], pairs / (np.mean(ms) * 1e-3), OPS_PER_PAIR_NF_AMP,
+                                 amp=True, kernel_ms=float(np.mean(ms)))}
 
 
 def bench_adjoint(args):
@@ -484,13 +508,13 @@ def bench_adjoint(args):
     wall, _ = timer.run(step, args.steps, per_step=False)
     h.forward(d, None, field, _lib.OUT_FIELD, ext)
     fwd_plan = h.plan()
-    # the adjoint call alone (pixel table, k_adjoint, finalize) on the last field, for the roofline of
+    # the adjoint call alone (pixel table, adjoint kernel, finalize) on the last field, for the roofline of
     # its dominant kernel
     _, ms_adj = StepTimer().run(lambda: h.adjoint_l2(d, field, target32, None, ext, want_amp=False), args.steps)
     adj_ms = float(np.mean(ms_adj))
-    roof = roofline_valu(_lib, load_mix("adjoint", 0), n * n0 * n1 / (adj_ms * 1e-3), OPS_PER_PAIR_ADJ,
+    roof = roofline(_lib, "adjoint", h.plan()["tile"], n * n0 * n1 / (adj_ms * 1e-3), OPS_PER_PAIR_ADJ,
                          kernel_ms=adj_ms)
-    roof["kernel_ms_note"] = "the adjoint call: pixel table, k_adjoint and its finalize"
+    roof["kernel_ms_note"] = "the adjoint call: pixel table, adjoint kernel and its finalize"
     log("roofline", roof)
     # the gradients of one step against long-double central differences of the loss (h = 1e-4 nm for
     # positions, 1e-4 rad for phases) on 24 position and 8 phase coordinates, and against the FP64

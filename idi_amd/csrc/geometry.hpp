@@ -342,8 +342,8 @@ struct WorkItem {
 
 // Pixel-tile variants.  0..3: VALU kernels, lanes form a 16 x 16 grid and each
 // lane owns PX x PY pixels (16x16, 16x32, 32x32, 32x64 pixels per workgroup).
-// 4: reserved (a matrix-core variant was measured 12% slower than the VALU tiles and
-// is not built: the phase is a nonlinear distance, not a contraction).
+// 4: reserved (forming the phase itself on the matrix cores was measured 12% slower than the
+// VALU tiles and is not built; tiles 17 on form the sums there).
 // 5, 6: mirror-pair VALU kernels (one or two 2 x 2 quads per lane; 32x32 and
 // 32x64 pixels per workgroup), which share one sincos per quad and emitter.
 // 7: mirror pairs with a centre per pair (one quad per lane, 32x32 pixels): the

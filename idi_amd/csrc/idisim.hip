@@ -1298,9 +1298,10 @@ static int adjoint_call(const char* who, idisim_handle* h, const double* emitter
     bool w = false;
     const Geom gl = split_geom(h, adj_tile, &w);
     const bool lam = w && !gl.nf;
-    // The separable form wherever its squares meet the bound: faster from the smallest sizes on (a
-    // call at 16^2 x 1 34 -> 24 us; the kernel at 256^2 x 4096 68 -> 42 us, at 512^2 x 20000 1880 -> 470).  Squares of 32 pixels take 0.6 of the time per
-    // pair of those of 16, where their workgroups fill the device.
+    // The separable form wherever its squares meet the bound: faster from the smallest sizes on (a call
+    // at 16^2 x 1 34 -> 24 us; the kernel at 256^2 x 4096 68 -> 42 us, at 512^2 x 20000 1880 -> 470).
+    // Squares of 32 pixels take 0.6 of the time per pair of those of 16, where their workgroups fill the
+    // device.
     const bool want_amp = grad_amp != nullptr;
     bool ws = false;
     const Geom gs = split_geom(h, kTileSep32V, &ws);

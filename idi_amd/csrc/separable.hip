@@ -16,9 +16,10 @@
 // The sums without a remainder keep FP32's precision: X and Y are formed in FP32 and split into two
 // FP16 parts each (22 bits; X_hi Y_hi + X_hi Y_lo + X_lo Y_hi, the products exact, the sums in FP32).
 // The split by itself costs 7e-8 relative L2.  The remainder's sums are weighted by M and need 1e-3
-// of that: the high parts alone (variant 22, whose M is ten times as large, splits the one along mu).  The image of 100000 emitters on 512 x 512 pixels is within 6.9e-7
-// of 64 bits (7.5e-7 with the mirror pairs of variant 13), 12345 emitters on 333 x 211 in the far
-// field within 4.6e-7 (6.2e-7).
+// of that: the high parts alone (variant 22, whose M is ten times as large, splits the one along mu).
+// The image of 100000 emitters on 512 x 512 pixels is within 6.9e-7 and 6.8e-7 of 64 bits at two draws
+// (7.5e-7 and 6.1e-7 with the mirror pairs of variant 13), 12345 emitters on 333 x 211 in the far field
+// within 4.6e-7 (6.2e-7).
 //
 // A wave owns one rectangle.  v_mfma_f32_32x32x16_f16 (16x16x32 for T = 16) takes 8 (16) emitters per
 // instruction as K = (re, im) pairs; lane l holds row l % T of X and column l % T of Y for 4 of them,
