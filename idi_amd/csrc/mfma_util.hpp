@@ -40,22 +40,26 @@ struct SepTraits<16> {
     static __device__ __forceinline__ int row(int i, int g) { return 4 * g + i; }
 };
 
-// (c, s) as FP16 pairs: h rounded to nearest, l the remainder rounded to nearest.
+// (c, s) as FP16 pairs: h rounded to nearest, l the remainder (exact in FP32) rounded to nearest.
+// No instruction that writes an operand stands in an asm (the empty ones write none): the compiler keeps
+// the wait states in front of a matrix instruction only for writers that it sees.  `one`, hidden from it, keeps a remainder one fused
+// multiply-add that rounds to FP16 itself (v_fma_mix), where a difference would take two instructions.
 __device__ __forceinline__ void split_half(float c, float s, half2_t& h, half2_t& l)
 {
     h = __builtin_convertvector((float2_t{c, s}), half2_t);
-    asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mixhi_f16 %0, -%1, 1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-        : "=&v"(l)
-        : "v"(h), "v"(c), "v"(s));
+    float one = 1.f;
+    asm("" : "+s"(one));
+    l = half2_t{(_Float16)__builtin_fmaf(-(float)h.x, one, c), (_Float16)__builtin_fmaf(-(float)h.y, one, s)};
+    asm("" : "+v"(l));  // rot90 turns the pair, and does not form it anew in the other order
 }
 
-// (x, y) -> (-y, x)
+// (x, y) -> (-y, x): one v_pk_mul_f16 that reads v turned (the factors are hidden as above, or the turn
+// would become an instruction of its own)
 __device__ __forceinline__ half2_t rot90(half2_t v)
 {
-    half2_t r;
-    asm("v_pk_mul_f16 %0, %1, 1.0 op_sel:[1,0] op_sel_hi:[0,0] neg_lo:[1,0]" : "=v"(r) : "v"(v));
-    return r;
+    unsigned sign = 0x3c00bc00u;  // (-1, 1)
+    asm("" : "+s"(sign));
+    return half2_t{v.y, v.x} * __builtin_bit_cast(half2_t, sign);
 }
 
 }  // namespace idisim
