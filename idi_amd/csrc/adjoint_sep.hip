@@ -171,7 +171,7 @@ __global__ __launch_bounds__(kAdjTile) void k_adj_sep_pixels(Geom g, const float
             if (l == 0 && tile) loss_tile[(size_t)(tx / 16) * tiles_y + ty / 16] = red[0];
         }
     }
-    // the power of two that brings the largest weight to [1/2, 1) (weights that are not finite or all
+    // the power of two that brings the largest weight to [2^13, 2^14) (weights that are not finite or all
     // zero: no scale)
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kAdjTile) void k_adj_sep_pixels(Geom g, const float
     m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     float sc = 1.f, back = 1.f;
     if (m > 0.f && m < INFINITY) {
-        const int ex = min(max(ilogbf(m) + 1, -120), 120);
+        const int ex = min(max(ilogbf(m) + 1 - kHalfTop, -120), 120);
         sc = ldexpf(1.f, -ex);
         back = ldexpf(1.f, ex);
     }

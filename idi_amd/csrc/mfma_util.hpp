@@ -40,6 +40,14 @@ struct SepTraits<16> {
     static __device__ __forceinline__ int row(int i, int g) { return 4 * g + i; }
 };
 
+// Amplitudes and weights are scaled by the power of two that brings the largest of a range to
+// [2^(kHalfTop - 1), 2^kHalfTop) before they are split.  FP16's smallest step is 2^-24 whatever the value, so
+// what the two parts leave of a value is 2^-23 of itself down to 2^-16 of the largest, and 2^-39 of the
+// largest below.  Scaled to [1/2, 1) it was 2^-25 of the largest: 1.5e-6 to 2.1e-6 of the field of 100000 emitters
+// of 1 beside one of 1000, and 6e-7 to 1e-6 of the gradients with one bright pixel a square, where FP32
+// phasors and weights leave 3.6e-7.
+constexpr int kHalfTop = 14;
+
 // (c, s) as FP16 pairs: h rounded to nearest, l the remainder (exact in FP32) rounded to nearest.
 // No instruction that writes an operand stands in an asm (the empty ones write none): the compiler keeps
 // the wait states in front of a matrix instruction only for writers that it sees.  `one`, hidden from it, keeps a remainder one fused

@@ -269,7 +269,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
         }
     }
 
-    // amplitudes: scaled by the power of two that brings the largest of the range to [1/2, 1)
+    // amplitudes: scaled by the power of two that brings the largest of the range to [2^13, 2^14)
     float ascale = 1.f, aback = 1.f;
     if (HAS_AMP && amp != nullptr) {
         float m = 0.f;
@@ -280,7 +280,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
         __syncthreads();
         m = fmaxf(fmaxf(s.amax[0], s.amax[1]), fmaxf(s.amax[2], s.amax[3]));
         if (m > 0.f && m < INFINITY) {
-            const int ex = min(max(ilogbf(m) + 1, -120), 120);
+            const int ex = min(max(ilogbf(m) + 1 - kHalfTop, -120), 120);
             ascale = ldexpf(1.f, -ex);
             aback = ldexpf(1.f, ex);
         }
