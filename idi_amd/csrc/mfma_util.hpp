@@ -50,14 +50,20 @@ constexpr int kHalfTop = 14;
 
 // (c, s) as FP16 pairs: h rounded to nearest, l the remainder (exact in FP32) rounded to nearest.
 // No instruction that writes an operand stands in an asm (the empty ones write none): the compiler keeps
-// the wait states in front of a matrix instruction only for writers that it sees.  `one`, hidden from it, keeps a remainder one fused
-// multiply-add that rounds to FP16 itself (v_fma_mix), where a difference would take two instructions.
+// the wait states in front of a matrix instruction only for writers that it sees.  `one`, hidden from it,
+// keeps a remainder one instruction (v_fma_mix_f32 reads h as it is).  MIX: v_fma_mixlo/hi_f16 round it as
+// well; otherwise both are packed by one conversion, as each write of half a register costs its reader a
+// wait.  100000 emitters on 512 x 512: 1.068 ms with MIX, 1.042 without; with amplitudes, where the
+// products fill the waits, 78.4 ms without and 77.4 with it (two shots of 1e6 on 1024 x 1024).
+template <bool MIX = false>
 __device__ __forceinline__ void split_half(float c, float s, half2_t& h, half2_t& l)
 {
     h = __builtin_convertvector((float2_t{c, s}), half2_t);
     float one = 1.f;
     asm("" : "+s"(one));
-    l = half2_t{(_Float16)__builtin_fmaf(-(float)h.x, one, c), (_Float16)__builtin_fmaf(-(float)h.y, one, s)};
+    float lc = __builtin_fmaf(-(float)h.x, one, c), ls = __builtin_fmaf(-(float)h.y, one, s);
+    if (!MIX) asm("" : "+v"(lc), "+v"(ls));
+    l = __builtin_convertvector((float2_t{lc, ls}), half2_t);
     asm("" : "+v"(l));  // rot90 turns the pair, and does not form it anew in the other order
 }
 

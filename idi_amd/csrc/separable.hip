@@ -136,7 +136,7 @@ __device__ __forceinline__ void sep_gen(const SepRecs<S>& q, const float (&gx)[3
             c *= q.a[i];
             sn *= q.a[i];
         }
-        split_half(c, sn, f.xh.p[i], f.xl.p[i]);
+        split_half<AMP>(c, sn, f.xh.p[i], f.xl.p[i]);
         constexpr int k0 = S::Q2 ? 1 : 0;
         f.x1[k0].p[i] = f.xh.p[i] * half2_t{h0.x, h0.x};
         f.x1[k0 + 1].p[i] = f.xh.p[i] * half2_t{h0.y, h0.y};
@@ -150,7 +150,7 @@ __device__ __forceinline__ void sep_gen(const SepRecs<S>& q, const float (&gx)[3
             float u = gy[b][0] * r.x;
             u = fmaf(gy[b][1], r.y, u);
             u = fmaf(gy[b][2], r.z, u);
-            split_half(__builtin_amdgcn_cosf(u), -__builtin_amdgcn_sinf(u), f.yh[b].p[i], f.yl[b].p[i]);
+            split_half<AMP>(__builtin_amdgcn_cosf(u), -__builtin_amdgcn_sinf(u), f.yh[b].p[i], f.yl[b].p[i]);
             f.zh[b].p[i] = rot90(f.yh[b].p[i]);
             f.zl[b].p[i] = rot90(f.yl[b].p[i]);
         }
