@@ -337,14 +337,19 @@ int run_forward(idisim_handle* h, const FwdCall& c, int tile, int splits)
     return IDISIM_OK;
 }
 
-// The mirror-pair forward of c into float4 split partials [splits][npix] only (no finalize):
-// idisim_loss_grad_l2 sums them in its adjoint pixel stage.
+// The mirror-pair or separable forward of c into float4 split partials [splits][npix] only (no
+// finalize): idisim_loss_grad_l2 sums them in its adjoint pixel stage.
 int run_forward_partials(idisim_handle* h, const FwdCall& c, int tile, int splits, float4* partial)
 {
     bool w = false;
     const Geom gl = split_geom(h, tile, &w);
     const bool a = (c.amp != nullptr) || (h->g.nf && h->g.scale);
-    if (w) return fail(IDISIM_E_UNSUPPORTED, "the mirror-pair tiles need the curvature folded into A");
+    if (w) return fail(IDISIM_E_UNSUPPORTED, "the mirror-pair and separable tiles need the curvature folded into A");
+    if (tile_sep(tile)) {
+        if (h->summode != 0) return fail(IDISIM_E_UNSUPPORTED, "the separable tiles have no per-term Kahan mode");
+        IDISIM_HIP(launch_fwd_sep(tile, a, gl, c.emit, c.amp, c.n, splits, partial, nullptr, c.kind, c.st));
+        return IDISIM_OK;
+    }
     const float* tab = nullptr;
     if (int rc = pair_table(h, c, tile, &tab)) return rc;
     IDISIM_HIP(launch_fwd_pair(tile, a, gl, c.emit, c.amp, c.n, splits, tab, partial, nullptr, c.kind, c.st));
@@ -354,11 +359,10 @@ int run_forward_partials(idisim_handle* h, const FwdCall& c, int tile, int split
 // The separable tiles take a forward of at least kSepPairs emitter-pixel pairs (n rounded down to its
 // tuning bucket) where they meet the bound.  Intensities: from 1e8 on (1000 emitters on 128 x 128
 // pixels, 1.6e7 pairs, take 13 to 14 us either way; 2048 on 256 x 256, 1.3e8 pairs, 22 against 34 us;
-// 12345 on 333 x 211 79 against 144; 100000 on 512 x 512 1.07 against 3.29 ms).  Fields: from 5e8 on.
-// Between the two lines they would be faster as well (4096 on 256 x 256: 30 against 52 us), but a field
-// there stays on the tiles that idisim_loss_grad_l2 sums its loss from, so that it and
-// idisim_adjoint_l2 on it give that call's bits at the sizes of a fit: the FP64 loss follows the
-// field's rounding, and the loss must not change.
+// 12345 on 333 x 211 79 against 144; 100000 on 512 x 512 1.07 against 3.29 ms).  Fields, of idisim_forward
+// and of idisim_loss_grad_l2 alike: from 5e8 on.  Between the two lines they would be faster as well (4096
+// on 256 x 256: 30 against 52 us); but the FP64 loss of a fit follows its field's rounding (1.3e-7 from 64 bits
+// with these tiles, up to 3.9e-7 with the others), and fits of that size keep the loss that they had.
 constexpr double kSepPairsIntensity = 1e8, kSepPairsField = 5e8;
 
 // The separable candidates of a call in `tiles`, in place of the others: of each rectangle the one
@@ -1251,8 +1255,8 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
     return IDISIM_OK;
 }
 
-// The forward that idisim_loss_grad_l2 runs inside its adjoint call: its planned mirror-pair
-// tile and split; the field is summed from its partials (field may then be NULL: not stored).
+// The forward that idisim_loss_grad_l2 runs inside its adjoint call: its planned mirror-pair or
+// separable tile and split; the field is summed from its partials (field may then be NULL: not stored).
 struct FusedForward {
     FwdCall c;
     Choice ch;
@@ -1401,9 +1405,12 @@ int idisim_loss_grad_l2(idisim_handle* h, const double* emitters, const double* 
         fbuf = h->field_tmp;
     }
     // an FP64 fallback forward writes the complex64 field through its finalize (out_f32)
-    FusedForward fz{FwdCall{emitters, amplitudes, n, fbuf, IDISIM_OUT_FIELD, st, split_path, !split_path}, Choice{}};
+    FusedForward fz{FwdCall{emitters, amplitudes, n, fbuf, IDISIM_OUT_FIELD, st, split_path, !split_path,
+                            use_sep_tiles(h, n, IDISIM_OUT_FIELD, split_path, &tiles)},
+                    Choice{}};
     if (int rc = plan_choose(h, fz.c, tiles, fz.ch)) return rc;
-    const bool fused = split_path && tile_pair(fz.ch.tile) && fz.ch.tile != kTileBlock && fz.ch.split > 1;
+    const bool fused = split_path && ((tile_pair(fz.ch.tile) && fz.ch.tile != kTileBlock) || tile_sep(fz.ch.tile)) &&
+                       fz.ch.split > 1;
     if (!fused) {  // the forward with its own finalize, then idisim_adjoint_l2
         if (int rc = run_forward(h, fz.c, fz.ch.tile, fz.ch.split)) return rc;
         plan_record(h, fz.c, fz.ch);
