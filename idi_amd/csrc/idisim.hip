@@ -1191,18 +1191,10 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
     } else if (it != h->tuned.end() && has_tile(tiles, it->second.tile)) {
         ch = it->second;
     } else if (h->autotune) {
-        // time the candidates on at most ~2e11 pairs (2e10 for the FP64 kernels), every shot cut to the
-        // same share: the queue keeps its number of items, on which the choice depends (two shots of 1e6
-        // emitters on 1024 x 1024 pixels are 512 items of 64 x 64 pixels or 256 of 64 x 128)
-        const double cap = split_path ? 2e11 : 2e10;
-        const double share = std::min(1.0, cap / ((double)total * (double)h->g.n0 * (double)h->g.n1));
-        std::vector<int64_t> toff(offsets, offsets + nshots + 1);
-        if (share < 1.0)
-            for (int64_t s = 1; s <= nshots; ++s) {
-                const int64_t ns = offsets[s] - offsets[s - 1];
-                toff[s] = toff[s - 1] + std::min(ns, std::max<int64_t>((int64_t)(share * (double)ns), kChunk));
-            }
-        const int64_t tshots = nshots;
+        // time the candidates on at most ~2e11 pairs (2e10 for the FP64 kernels)
+        const std::vector<int64_t> toff =
+            tuning_offsets(offsets, nshots, (double)h->g.n0 * (double)h->g.n1, split_path ? 2e11 : 2e10);
+        const int64_t tshots = (int64_t)toff.size() - 1;
         Timer tm;
         double best = std::numeric_limits<double>::infinity();
         for (int v : tiles) {

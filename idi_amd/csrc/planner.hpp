@@ -501,6 +501,26 @@ inline std::vector<int> eligible_tiles(const Planner* h, double rho, double* bes
     return out;
 }
 
+// What the batched tuner times, as offsets: at most about `cap` pairs.  The shots that fill the queue (8192
+// items of 64 x 64 pixels, 32 workgroups a CU) are kept, each cut to the same share (not below a chunk, 9e9
+// pairs in all), because the choice depends on the number of items: two shots of 1e6 emitters on 1024 x 1024
+// pixels are 512 items of 64 x 64 or 256 of 64 x 128.  Beyond those a longer queue chooses alike, and
+// whole shots are added up to the cap only.
+inline std::vector<int64_t> tuning_offsets(const int64_t* offsets, int64_t nshots, double npix, double cap)
+{
+    constexpr double kQueuePixels = 8192.0 * 64 * 64;
+    int64_t ts = (int64_t)std::min((double)nshots, std::ceil(kQueuePixels / npix));
+    while (ts < nshots && (double)offsets[ts + 1] * npix <= cap) ++ts;
+    const double share = std::min(1.0, cap / std::max(1.0, (double)offsets[ts] * npix));
+    std::vector<int64_t> out(offsets, offsets + ts + 1);
+    if (share < 1.0)
+        for (int64_t s = 1; s <= ts; ++s) {
+            const int64_t ns = offsets[s] - offsets[s - 1];
+            out[s] = out[s - 1] + std::min(ns, std::max<int64_t>((int64_t)(share * (double)ns), kChunk));
+        }
+    return out;
+}
+
 // The separable tiles that meet the tolerance, the widest first.
 inline std::vector<int> eligible_sep_tiles(const Planner* h, double rho)
 {
