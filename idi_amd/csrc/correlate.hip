@@ -22,7 +22,7 @@
 #include <algorithm>
 #include <climits>
 
-#include "kernels.hpp"
+#include "device_util.hpp"
 
 namespace idisim {
 
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void k_qcorr_runs(const float* __restrict__ zd
             s_tgt[w][i] = make_float2(((float)c - yc) * z, z);
             s_tv[w][i] = img[(size_t)tr * nc + c];
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         float px = kQNone, py = 0.f, pz = 0.f, qx = kQNone, qy = 0.f, qz = 0.f;  // the open run's bin, the closed one's
         double acc = 0.0, closed = 0.0;
         auto add = [&]() {
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256) void k_qcorr_runs(const float* __restrict__ zd
         qz = pz;
         closed = acc;
         if (qx != kQNone) add();
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
     }
     __syncthreads();
     for (int b = threadIdx.x; b < wx * wy * wz; b += blockDim.x) {

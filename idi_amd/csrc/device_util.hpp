@@ -20,6 +20,15 @@ __device__ __forceinline__ void kahan_add_d(double& sum, double& comp, double v)
     sum = t;
 }
 
+// Orders the LDS accesses of a wave's lanes: what any of them wrote before is read by all after.  The
+// hardware keeps a wave's LDS accesses in order; the fences (no instruction) hold the compiler to it.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Pixel-index centre of the part of a tile that lies on the detector.
 __device__ __forceinline__ void tile_centre(const Geom& g, int tx0, int ty0, int TX, int TY,
                                             double& cx, double& cy)
