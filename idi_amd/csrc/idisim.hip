@@ -53,7 +53,7 @@ int fail(int code, const std::string& msg)
 // larger emitter extent can push a tile's error bound past the tolerance).
 struct TuneKey {
     int kind, has_amp, batched, split_path, nbucket;
-    int sep;  // the separable tiles were candidates
+    int sep;  // whether the separable tiles were candidates (SepUse)
     bool operator<(const TuneKey& o) const
     {
         return std::tie(kind, has_amp, batched, split_path, nbucket, sep) <
@@ -229,6 +229,9 @@ Geom split_geom(const idisim_handle* h, int tile, bool* w)
 }
 
 // ------------------------------ single shot --------------------------------
+// Whether the separable tiles are a call's candidates: not at all, in place of the others, or beside them.
+enum SepUse { kSepNone = 0, kSepOnly = 1, kSepToo = 2 };
+
 struct FwdCall {
     const double* emit;
     const double* amp;
@@ -238,7 +241,7 @@ struct FwdCall {
     hipStream_t st;
     bool split_path;  // FP32-split kernels (false: FP64 kernels)
     bool out_f32;     // FP64 kernels writing a complex64 / float32 output (fallback)
-    bool sep = false; // the separable tiles are the candidates (use_sep_tiles)
+    SepUse sep = kSepNone;  // use_sep_tiles
     // fixed device scratch of idisim_forward_noalloc (nullptr: the handle's own, grown on demand)
     void* fixed = nullptr;
     size_t fixed_cap = 0;
@@ -365,25 +368,43 @@ int run_forward_partials(idisim_handle* h, const FwdCall& c, int tile, int split
 // with these tiles, up to 3.9e-7 with the others), and fits of that size keep the loss that they had.
 constexpr double kSepPairsIntensity = 1e8, kSepPairsField = 5e8;
 
-// The separable candidates of a call in `tiles`, in place of the others: of each rectangle the one
-// with the fewest sums.
-bool sep_candidates(const idisim_handle* h, std::vector<int>* tiles)
+// Emitters (of a batch: a shot on average) from which they take such a call.  They pay per rectangle (the
+// columns' frames, the mixed remainder's terms) whatever the number of emitters, so a shot of few emitters
+// is slower on them: 2000 x 2000 pixels with 32 emitters 33 against 37 us (37 against 59 where the 16 x 16
+// rectangles alone meet the bound), 64 52 against 42 (58 against 69), 96 on 1400 x 1400 38 against 27 (43
+// against 43); batches on 256 x 256 with 8 a shot 211 against 281 us (408), 32 155 against 137 (157
+// against 190), 64 78 against 63 (82 against 79), 128 73 against 53 (85 against 69).  Between the outer
+// two lines the tuner times them beside the others; without it the middle one holds.
+constexpr int kSepFewBucket = 5, kSepManyBucket = 7;  // 32 and 128 emitters (nbucket)
+constexpr int64_t kSepUntuned = 96;
+
+// The separable candidates of a call with n emitters a shot in `tiles`, in place of the others or after
+// them: of each rectangle the one with the fewest sums.
+SepUse sep_candidates(const idisim_handle* h, int64_t n, std::vector<int>* tiles)
 {
+    if (nbucket(n) < kSepFewBucket) return kSepNone;
     std::vector<int> sep;
     for (int v : eligible_sep_tiles(h, h->rho))
         if (sep.empty() || sep_shape(v) != sep_shape(sep.back())) sep.push_back(v);
-    if (sep.empty()) return false;
-    *tiles = sep;
-    return true;
+    if (sep.empty()) return kSepNone;
+    if (nbucket(n) >= kSepManyBucket) {
+        *tiles = sep;
+        return kSepOnly;
+    }
+    tiles->insert(tiles->end(), sep.begin(), sep.end());
+    return kSepToo;
 }
 
-bool use_sep_tiles(const idisim_handle* h, int64_t n, int kind, bool split_path, std::vector<int>* tiles)
+SepUse use_sep_tiles(const idisim_handle* h, int64_t n, int kind, bool split_path, std::vector<int>* tiles)
 {
-    if (!split_path || h->force_tile >= 0) return false;
+    if (!split_path || h->force_tile >= 0) return kSepNone;
     const double pairs = std::ldexp(1.0, nbucket(n)) * (double)h->g.n0 * (double)h->g.n1;
-    if (pairs < (kind == OUT_INTENSITY ? kSepPairsIntensity : kSepPairsField)) return false;
-    return sep_candidates(h, tiles);
+    if (pairs < (kind == OUT_INTENSITY ? kSepPairsIntensity : kSepPairsField)) return kSepNone;
+    return sep_candidates(h, n, tiles);
 }
+
+// Whether a call whose candidates are not timed takes one of them.
+bool sep_untuned(SepUse use, int64_t n) { return use == kSepOnly || (use == kSepToo && n >= kSepUntuned); }
 
 // Workgroups per CU that a heuristic split aims at: as many as are resident of the separable tiles.
 int64_t target_groups(const idisim_handle* h, int tile)
@@ -421,7 +442,7 @@ int heuristic_split(const idisim_handle* h, int64_t n, int tile)
 // candidate forwards into c.out), or the heuristic.
 int plan_choose(idisim_handle* h, const FwdCall& c, const std::vector<int>& tiles, Choice& ch)
 {
-    const TuneKey key{c.kind, c.amp != nullptr, 0, c.split_path ? 1 : 0, nbucket(c.n), c.sep ? 1 : 0};
+    const TuneKey key{c.kind, c.amp != nullptr, 0, c.split_path ? 1 : 0, nbucket(c.n), (int)c.sep};
     auto it = h->tuned.find(key);
     const bool forced = h->force_tile >= 0 || h->force_split > 0;
     if (forced) {
@@ -505,9 +526,11 @@ int plan_choose(idisim_handle* h, const FwdCall& c, const std::vector<int>& tile
     } else {
         // heuristic: a mirror-pair quad per lane if allowed (of the separable tiles the widest that can
         // fill the device), enough splits for 4 WG/CU (or all that are resident)
-        ch.tile = c.sep ? tiles.back() : tiles.front();
-        if (c.sep) {
+        const bool sep = sep_untuned(c.sep, c.n);
+        ch.tile = sep ? tiles.back() : tiles.front();
+        if (sep) {
             for (int v : tiles) {
+                if (!tile_sep(v)) continue;
                 const int64_t wgs = (int64_t)((h->g.n0 + tile_rows(v) - 1) / tile_rows(v)) *
                                     ((h->g.n1 + tile_cols(v) - 1) / tile_cols(v)) * ((c.n + kChunk - 1) / kChunk);
                 if (wgs >= 2 * target_groups(h, v)) {
@@ -599,7 +622,7 @@ struct BatchCall {
     int kind;
     hipStream_t st;
     bool split_path;
-    bool sep = false;  // the separable tiles are the candidates
+    SepUse sep = kSepNone;  // sep_candidates
 };
 
 int launch_batched(idisim_handle* h, const BatchCall& c, int tile, int blocks_per_cu, hipStream_t st)
@@ -1172,15 +1195,15 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
         return IDISIM_OK;
     }
     BatchCall c{emitters, amplitudes, out, out_kind, st, split_path};
+    const int64_t per_shot = std::max<int64_t>(1, total / nshots);
     // the separable tiles from 1e8 pairs on: 40 shots of 20 to 60 emitters take 48 against 45 us on
     // 128 x 128 pixels (2.6e7 pairs) and 52 against 64 us on 256 x 256 (1e8); 64 shots of 1000 to 50000 on
-    // 256 x 256 8.6 against 16.3 ms
+    // 256 x 256 8.8 against 17.3 ms
     if (split_path && h->force_tile < 0 &&
         (double)total * (double)h->g.n0 * (double)h->g.n1 >= kSepPairsIntensity)
-        c.sep = sep_candidates(h, &tiles);
+        c.sep = sep_candidates(h, per_shot, &tiles);
 
-    const TuneKey key{out_kind, amplitudes != nullptr, 1, split_path ? 1 : 0,
-                      nbucket(std::max<int64_t>(1, total / nshots)), c.sep ? 1 : 0};
+    const TuneKey key{out_kind, amplitudes != nullptr, 1, split_path ? 1 : 0, nbucket(per_shot), (int)c.sep};
     Choice ch;
     auto it = h->tuned.find(key);
     if (h->force_tile >= 0 || h->force_split > 0) {
@@ -1223,8 +1246,9 @@ int idisim_forward_batched(idisim_handle* h, const double* emitters, const doubl
         }
         h->tuned[key] = ch;
     } else {
-        ch.tile = c.sep ? tiles.back() : tiles.front();
-        if (!c.sep) {
+        const bool sep = sep_untuned(c.sep, per_shot);
+        ch.tile = sep ? tiles.back() : tiles.front();
+        if (!sep) {
             for (int v : {kTileRefL, kTileRef1, kTileRefC1, kTileRefSC, kTileRefS, kTileRef2, kTileRefC2, kTilePair1,
                           kTileBlock, kTilePairC, 2, 1, 3, 0})
                 if (has_tile(tiles, v)) {
