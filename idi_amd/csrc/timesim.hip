@@ -312,6 +312,7 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused(Geom g, const double* __re
         u.sorted.idx[tid * S + k] = (unsigned short)js[k];
     }
     __syncthreads();  // every lane reads its neighbours' first and last keys
+    const Tt top = u.sorted.key[(BLOCK - 1) * S + ITEMS - 1];  // a NaN key leaves the sort last, behind the padding
     const Tt* skey = u.sorted.key + tid * S;
     const unsigned short* sidx = u.sorted.idx + tid * S;
     const int64_t i0 = (int64_t)tid * ITEMS;
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused(Geom g, const double* __re
     double A = 0.0, Br = 0.0, Bi = 0.0, C = 0.0;
 #pragma unroll 1
     for (int k = 0; k < cnt; ++k) {
-        const int j = sidx[k];
+        const int j = min((int)sidx[k], (int)n - 1);  // (then the padding's indices are among the first n)
         double re, im;
         arrival_amp<sizeof(Tt) == 4>(g, r, R, emit + 4 * (int64_t)j, &re, &im);
         const double tk = (double)skey[k];
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused(Geom g, const double* __re
         if (tid < s2) ssum[tid] += ssum[tid + s2];
         __syncthreads();
     }
-    if (tid == 0) out[p] = ssum[0] * (0.5 * tau);
+    if (tid == 0) out[p] = top != top ? NAN : ssum[0] * (0.5 * tau);
 }
 
 // k_time_fused where an amplitude is its phase alone (float32 keys, no 1/r): the FP32 phase goes through
@@ -434,6 +435,7 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused_phase(Geom g, const double
     const int cnt = (int)(n - i0 < ITEMS ? (n - i0 > 0 ? n - i0 : 0) : ITEMS);
     const double tprev = tid > 0 ? (double)u.scan.last[tid - 1] : (double)key[0];
     const double tnext = tid + 1 < BLOCK ? (double)u.scan.first[tid + 1] : 0.0;
+    const float top = u.scan.last[BLOCK - 1];  // a NaN key leaves the sort last, behind the padding
 
     // the sums A, B, C of k_time_fused
     double pr = 0.0, pi = 0.0, D = 1.0, tl = tprev, A = 0.0, Br = 0.0, Bi = 0.0, C = 0.0;
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(BLOCK) void k_time_fused_phase(Geom g, const double
         if (tid < s2) u.sum[tid] += u.sum[tid + s2];
         __syncthreads();
     }
-    if (tid == 0) out[p] = u.sum[0] * (0.5 * tau);
+    if (tid == 0) out[p] = top != top ? NAN : u.sum[0] * (0.5 * tau);
 }
 
 template <typename Tt>
