@@ -184,6 +184,13 @@ __global__ __launch_bounds__(kAdjTile) void k_adj_sep_pixels(Geom g, const float
         sc = ldexpf(1.f, -ex);
         back = ldexpf(1.f, ex);
     }
+    // The matrix instruction truncates its sums downwards; from square to square the weights' sign changes
+    // and that bias cancels (phase gradients of 2000 x 2000 pixels 9.2e-7 from 64 bits without it, 3.2e-7 of
+    // k_adjoint).
+    if ((sx / T + sy / T) & 1) {
+        sc = -sc;
+        back = -back;
+    }
     constexpr float hw = 0.5f * (T - 1);
     const double cx = sx + (double)hw, cy = sy + (double)hw;
     const SqAxes ax = sq_axes(g, cx, cy, T);

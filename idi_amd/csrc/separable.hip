@@ -226,10 +226,15 @@ __device__ __forceinline__ void sep_pixel(int tx0, int ty0, int w, int l, int i,
 }
 
 // The sums of the workgroup's 2 x 2 rectangles over emitters [e0, e1), into o (sep_pixel's order).
+//
+// The instruction truncates its sums of eight products downwards: 7e-10 per emitter in both parts of the
+// field, which grows with the number of emitters (1.1e-6 of the field of 1e6, where the mirror-pair
+// tiles have 3.8e-7).  So the sign of X changes from one merge interval to the next (and from one split to
+// the next: `split`), and with it that of what is merged; X's weights for the remainder's sums change too.
 template <class S, bool HAS_AMP>
 __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict__ emit,
-                                         const double* __restrict__ amp, int64_t e0, int64_t e1, int tx0, int ty0,
-                                         SepLds<S>& s, SepOut<S>& o)
+                                         const double* __restrict__ amp, int64_t e0, int64_t e1, int split, int tx0,
+                                         int ty0, SepLds<S>& s, SepOut<S>& o)
 {
     constexpr int T = S::T, NB = S::NB, R = S::R, NE = S::NE;
     constexpr bool Q2 = S::Q2;
@@ -303,7 +308,8 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
         }
     }
 
-    for (int64_t m0 = e0; m0 < e1; m0 += kSepMerge) {
+    float sign = (split & 1) ? -1.f : 1.f;
+    for (int64_t m0 = e0; m0 < e1; m0 += kSepMerge, sign = -sign) {
         const int64_t m1 = m0 + kSepMerge < e1 ? m0 + kSepMerge : e1;
         float npad = 0.f;
         for (int64_t base = m0; base < m1; base += S::kStage) {
@@ -320,6 +326,8 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
                     const double* a4 = emit + 4 * e;
                     const double ea = (HAS_AMP && amp != nullptr) ? amp[e] : 1.0;
                     r = make_split_rec(g, c, a4[0], a4[1], a4[2], a4[3], ea);
+                    // half a revolution, within [-1/2, 1/2] as A itself
+                    if (!HAS_AMP && sign < 0.f) r.A -= copysignf(0.5f, r.A);
                 } else if (!HAS_AMP) {
                     // the last steps' missing emitters: at the origin, with phases 0 and 1/2 in turn,
                     // +1 and -1 in every pixel; an odd one is taken off below
@@ -327,24 +335,25 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
                 }
                 const float x = r.x * g.sepscale, y = r.y * g.sepscale, z = r.z * g.sepscale;
                 s.r[j] = make_float4(x, y, z, r.A);
+                const float hx = sign * x, hy = sign * y, hz = sign * z;
                 if constexpr (S::kBasis) {
                     constexpr int k0 = Q2 ? 1 : 0;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const float(*d)[3] = s.b[v];
-                        s.h[v][j] = half2_t{(_Float16)(d[k0][0] * x + d[k0][1] * y + d[k0][2] * z),
-                                            (_Float16)(d[k0 + 1][0] * x + d[k0 + 1][1] * y + d[k0 + 1][2] * z)};
+                        s.h[v][j] = half2_t{(_Float16)(d[k0][0] * hx + d[k0][1] * hy + d[k0][2] * hz),
+                                            (_Float16)(d[k0 + 1][0] * hx + d[k0 + 1][1] * hy + d[k0 + 1][2] * hz)};
                         if constexpr (Q2) {
-                            const float q = d[0][0] * x + d[0][1] * y + d[0][2] * z;
+                            const float q = d[0][0] * hx + d[0][1] * hy + d[0][2] * hz;
                             s.c[v][j] = q;
-                            s.c2[v][j] = half2_t{(_Float16)(q * q), (_Float16)(q * q)};
+                            s.c2[v][j] = half2_t{(_Float16)(sign * q * q), (_Float16)(sign * q * q)};
                         }
                     }
                 } else {
-                    s.h[0][j] = half2_t{(_Float16)x, (_Float16)y};
-                    s.h[1][j] = half2_t{(_Float16)z, (_Float16)z};
+                    s.h[0][j] = half2_t{(_Float16)hx, (_Float16)hy};
+                    s.h[1][j] = half2_t{(_Float16)hz, (_Float16)hz};
                 }
-                if (HAS_AMP) s.amp[j] = r.amp * ascale;
+                if (HAS_AMP) s.amp[j] = r.amp * (sign * ascale);
             }
             if (!HAS_AMP) npad = (float)((pad - cnt) & 1);
             __syncthreads();
@@ -380,7 +389,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
             for (int i = 0; i < R; ++i) {
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    const float v = p ? acc.e0[b][p][i] : acc.e0[b][p][i] - npad;
+                    const float v = sign * (p ? acc.e0[b][p][i] : acc.e0[b][p][i] - npad);
                     acc.e0[b][p][i] = 0.f;
                     float sum = o.at(p, b * R + i), cmp = o.at(2 + p, b * R + i);
                     kahan_add(sum, cmp, v);
@@ -443,7 +452,7 @@ __global__ __launch_bounds__(kBlock, S::kWaves) void k_fwd_sep(Geom g, const dou
     const int64_t e0 = (int64_t)blockIdx.y * per_split;
     const int64_t e1 = (e0 + per_split < n) ? e0 + per_split : n;
     SepOut<S> o;
-    sep_tile<S, HAS_AMP>(g, emit, amp, e0, e1, tx0, ty0, s, o);
+    sep_tile<S, HAS_AMP>(g, emit, amp, e0, e1, blockIdx.y, tx0, ty0, s, o);
     const Geom gs = item_geom();  // store frames formed here (see k_batched_pair)
     const size_t npix = (size_t)gs.n0 * gs.n1;
 #pragma unroll S::kStoreUnroll
@@ -482,7 +491,7 @@ __global__ __launch_bounds__(kBlock, S::kWaves) void k_batched_sep(Geom g0, cons
         const Geom g = item_geom();
         const int tx0 = (wi.tile / tiles_y) * S::kRows, ty0 = (wi.tile % tiles_y) * S::kCols;
         SepOut<S> o;
-        sep_tile<S, HAS_AMP>(g, emit, amp, wi.e0, wi.e1, tx0, ty0, s, o);
+        sep_tile<S, HAS_AMP>(g, emit, amp, wi.e0, wi.e1, 0, tx0, ty0, s, o);
         char* outs = static_cast<char*>(out) +
                      (size_t)wi.shot * npix * (kind == OUT_INTENSITY ? sizeof(float) : sizeof(float2));
         const Geom gs = item_geom();  // as in k_batched_pair
