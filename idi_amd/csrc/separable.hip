@@ -37,10 +37,11 @@
 namespace idisim {
 
 namespace {
-// Emitters between two merges of the FP32 sums into the compensated ones.  An instruction adds the
-// products of 8 or 16 emitters before it rounds into its sum, so 512 emitters see no more roundings
-// than the 256 single additions of the other tiles.
-constexpr int kSepMerge = 512;
+// Emitters between two merges of the FP32 sums into the long ones, as in the other tiles.  A step of 8 or 16
+// emitters rounds into its sum six times: with 512 emitters an image of random phases is 4.0e-7 off 64 bits,
+// with 256 3.1e-7 (the mirror-pair tiles 3.2e-7), with 128 2.5e-7 in 3% more time.
+constexpr int kSepMerge = kChunk;
+static_assert(kSepMerge % kBlock == 0, "a lane's staged emitters share the sign of their merge interval");
 
 // Shape of a kernel.  T: rows of a wave's rectangle and columns of its NB blocks (T x NB T pixels);
 // NE: directions along which the mixed remainder is kept (3: all; 2: sep_basis_of); Q2: for larger
@@ -53,7 +54,7 @@ struct SepShape {
     static constexpr int R = SepTraits<T>::kRegs, kStep = SepTraits<T>::kStep;
     static constexpr int kRows = 2 * T, kCols = 2 * T * NB;  // workgroup tile: 2 x 2 waves
     static constexpr bool kBasis = NE == 2 || Q2;  // the remainder along the wave's own directions
-    static constexpr bool kLdsSums = T == 32;  // compensated sums in LDS (registers hold only T = 16's)
+    static constexpr bool kLdsSums = T == 32;  // long sums in LDS (registers hold only T = 16's)
     static constexpr int kStoreUnroll = kLdsSums ? 1 : NB * R;  // the FP64 store is long
     // emitters staged at a time: two per lane where one workgroup fills a CU, so that the FP64 chains of
     // two records overlap
@@ -69,8 +70,7 @@ struct SepAcc {
     typename SepTraits<S::T>::acc_t e2[S::NB][2];         // sum (mu' . r')^2 X Y (Q2)
 };
 
-// LDS of a workgroup: the staged emitters and, for T = 32, the compensated sums (64 or 128 floats per
-// lane).
+// LDS of a workgroup: the staged emitters and, for T = 32, the long sums in FP64 (32 or 64 per lane).
 template <class S>
 struct SepLds {
     float4 r[S::kSlots];  // r' (scaled), A
@@ -80,7 +80,7 @@ struct SepLds {
     float amp[S::kSlots];
     float c[S::Q2 ? 4 : 1][S::Q2 ? S::kSlots : 1];     // mu' . r' of each wave
     half2_t c2[S::Q2 ? 4 : 1][S::Q2 ? S::kSlots : 1];  // its square, twice
-    float k[S::kLdsSums ? 4 : 1][S::kLdsSums ? 4 * S::NB * S::R : 1][64];
+    double k[S::kLdsSums ? 4 : 1][S::kLdsSums ? 2 * S::NB * S::R : 1][64];
     float amax[4];
     float b[4][3][3];  // orthonormal directions of each wave's rectangle, mu / |mu| first
 };
@@ -202,18 +202,55 @@ __device__ __forceinline__ void sep_interleave()
     }
 }
 
-// The four words of a pixel (re, im and their compensations), of block b and register i.
+// The long sums of a lane's pixels, word i = b R + register of block b, part p (re, im).  T = 16: FP32 with
+// compensations in registers; T = 32: FP64 in LDS, added to without reading them back (ds_add_f64; four
+// words read, compensated and written cost 1.151 against 1.040 ms for 100000 emitters on 512 x 512).
 template <class S>
 struct SepOut {
-    float v[S::kLdsSums ? 1 : 4][S::NB * S::R];
-    float (*k)[64];
+    static constexpr int N = S::NB * S::R;
+    float v[S::kLdsSums ? 1 : 4][N];
+    double (*k)[64];
     int l;
-    __device__ __forceinline__ float& at(int word, int i)
+    __device__ __forceinline__ void clear(int p, int i)
     {
         if constexpr (S::kLdsSums)
-            return k[word * S::NB * S::R + i][l];
+            k[p * N + i][l] = 0.0;
         else
-            return v[word][i];
+            v[p][i] = v[2 + p][i] = 0.f;
+    }
+    __device__ __forceinline__ void add(int p, int i, float x)
+    {
+        if constexpr (S::kLdsSums)
+            (void)__hip_atomic_fetch_add(&k[p * N + i][l], (double)x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        else
+            kahan_add(v[p][i], v[2 + p][i], x);
+    }
+    __device__ __forceinline__ void scale(int p, int i, float f)  // by a power of two
+    {
+        if constexpr (S::kLdsSums) {
+            k[p * N + i][l] *= (double)f;
+        } else {
+            v[p][i] *= f;
+            v[2 + p][i] *= f;
+        }
+    }
+    __device__ __forceinline__ double value(int p, int i) const
+    {
+        if constexpr (S::kLdsSums)
+            return k[p * N + i][l];
+        else
+            return (double)v[p][i] - (double)v[2 + p][i];
+    }
+    // the sum and its compensation, as the split partials hold them (value = x - y)
+    __device__ __forceinline__ float2 parts(int p, int i) const
+    {
+        if constexpr (S::kLdsSums) {
+            const double d = k[p * N + i][l];
+            const float sum = (float)d;
+            return make_float2(sum, (float)((double)sum - d));
+        } else {
+            return make_float2(v[p][i], v[2 + p][i]);
+        }
     }
 };
 
@@ -303,75 +340,93 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
                 if (Q2) acc.e2[b][p][i] = 0.f;
 #pragma unroll
                 for (int k = 0; k < NE; ++k) acc.e1[b][k][p][i] = 0.f;
-                o.at(p, b * R + i) = o.at(2 + p, b * R + i) = 0.f;
+                o.clear(p, b * R + i);
             }
         }
     }
 
-    float sign = (split & 1) ? -1.f : 1.f;
-    for (int64_t m0 = e0; m0 < e1; m0 += kSepMerge, sign = -sign) {
-        const int64_t m1 = m0 + kSepMerge < e1 ? m0 + kSepMerge : e1;
-        float npad = 0.f;
-        for (int64_t base = m0; base < m1; base += S::kStage) {
-            const int cnt = (m1 - base) < (int64_t)S::kStage ? (int)(m1 - base) : S::kStage;
-            const int pad = (cnt + 2 * S::kStep - 1) / (2 * S::kStep) * (2 * S::kStep);
-            __syncthreads();  // the previous emitters have been consumed by every lane
+    // the long sums take what the accumulators hold, without `npad` padding emitters, and these start anew
+    auto merge = [&](float sign, float npad) {
 #pragma unroll
-            for (int q = 0; q < S::kStage; q += kBlock) {
-                const int j = q + tid;
-                if (j >= pad) break;
-                SplitRec r = {};
-                if (j < cnt) {
-                    const int64_t e = base + j;
-                    const double* a4 = emit + 4 * e;
-                    const double ea = (HAS_AMP && amp != nullptr) ? amp[e] : 1.0;
-                    r = make_split_rec(g, c, a4[0], a4[1], a4[2], a4[3], ea);
-                    // half a revolution, within [-1/2, 1/2] as A itself
-                    if (!HAS_AMP && sign < 0.f) r.A -= copysignf(0.5f, r.A);
-                } else if (!HAS_AMP) {
-                    // the last steps' missing emitters: at the origin, with phases 0 and 1/2 in turn,
-                    // +1 and -1 in every pixel; an odd one is taken off below
-                    r.A = ((j - cnt) & 1) ? 0.5f : 0.f;
-                }
-                const float x = r.x * g.sepscale, y = r.y * g.sepscale, z = r.z * g.sepscale;
-                s.r[j] = make_float4(x, y, z, r.A);
-                const float hx = sign * x, hy = sign * y, hz = sign * z;
-                if constexpr (S::kBasis) {
-                    constexpr int k0 = Q2 ? 1 : 0;
+        for (int b = 0; b < NB; ++b) {
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const float(*d)[3] = s.b[v];
-                        s.h[v][j] = half2_t{(_Float16)(d[k0][0] * hx + d[k0][1] * hy + d[k0][2] * hz),
-                                            (_Float16)(d[k0 + 1][0] * hx + d[k0 + 1][1] * hy + d[k0 + 1][2] * hz)};
-                        if constexpr (Q2) {
-                            const float q = d[0][0] * hx + d[0][1] * hy + d[0][2] * hz;
-                            s.c[v][j] = q;
-                            s.c2[v][j] = half2_t{(_Float16)(sign * q * q), (_Float16)(sign * q * q)};
-                        }
-                    }
-                } else {
-                    s.h[0][j] = half2_t{(_Float16)hx, (_Float16)hy};
-                    s.h[1][j] = half2_t{(_Float16)hz, (_Float16)hz};
+            for (int i = 0; i < R; ++i) {
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    o.add(p, b * R + i, sign * (p ? acc.e0[b][p][i] : acc.e0[b][p][i] - npad));
+                    acc.e0[b][p][i] = 0.f;
                 }
-                if (HAS_AMP) s.amp[j] = r.amp * (sign * ascale);
             }
-            if (!HAS_AMP) npad = (float)((pad - cnt) & 1);
-            __syncthreads();
-            if (!active) continue;
-            SepFrags<S> f0, f1;
-            SepRecs<S> q0, q1;
+        }
+    };
+    // X's sign of an emitter: that of its merge interval
+    auto sign_of = [&](int64_t e) { return (((e - e0) / kSepMerge + split) & 1) ? -1.f : 1.f; };
+
+    for (int64_t base = e0; base < e1; base += S::kStage) {
+        const int cnt = (e1 - base) < (int64_t)S::kStage ? (int)(e1 - base) : S::kStage;
+        const int pad = (cnt + 2 * S::kStep - 1) / (2 * S::kStep) * (2 * S::kStep);
+        __syncthreads();  // the previous emitters have been consumed by every lane
+#pragma unroll
+        for (int q = 0; q < S::kStage; q += kBlock) {
+            const int j = q + tid;
+            if (j >= pad) break;
+            const float sign = sign_of(base + q);
+            SplitRec r = {};
+            if (j < cnt) {
+                const int64_t e = base + j;
+                const double* a4 = emit + 4 * e;
+                const double ea = (HAS_AMP && amp != nullptr) ? amp[e] : 1.0;
+                r = make_split_rec(g, c, a4[0], a4[1], a4[2], a4[3], ea);
+                // half a revolution, within [-1/2, 1/2] as A itself
+                if (!HAS_AMP && sign < 0.f) r.A -= copysignf(0.5f, r.A);
+            } else if (!HAS_AMP) {
+                // the last steps' missing emitters: at the origin, with phases 0 and 1/2 in turn,
+                // +1 and -1 in every pixel; an odd one is taken off below
+                r.A = ((j - cnt) & 1) ? 0.5f : 0.f;
+            }
+            const float x = r.x * g.sepscale, y = r.y * g.sepscale, z = r.z * g.sepscale;
+            s.r[j] = make_float4(x, y, z, r.A);
+            const float sx = sign * x, sy = sign * y, sz = sign * z;
+            if constexpr (S::kBasis) {
+                constexpr int k0 = Q2 ? 1 : 0;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float(*d)[3] = s.b[v];
+                    s.h[v][j] = half2_t{(_Float16)(d[k0][0] * sx + d[k0][1] * sy + d[k0][2] * sz),
+                                        (_Float16)(d[k0 + 1][0] * sx + d[k0 + 1][1] * sy + d[k0 + 1][2] * sz)};
+                    if constexpr (Q2) {
+                        const float q1 = d[0][0] * sx + d[0][1] * sy + d[0][2] * sz;
+                        s.c[v][j] = q1;
+                        s.c2[v][j] = half2_t{(_Float16)(sign * q1 * q1), (_Float16)(sign * q1 * q1)};
+                    }
+                }
+            } else {
+                s.h[0][j] = half2_t{(_Float16)sx, (_Float16)sy};
+                s.h[1][j] = half2_t{(_Float16)sz, (_Float16)sz};
+            }
+            if (HAS_AMP) s.amp[j] = r.amp * (sign * ascale);
+        }
+        const float npad = HAS_AMP ? 0.f : (float)((pad - cnt) & 1);
+        __syncthreads();
+        if (!active) continue;
+        SepFrags<S> f0, f1;
+        SepRecs<S> q0, q1;
+        if constexpr (T == 32) {
+            // the operands of a step are formed during the matrix instructions of the step before
+            // (past the last step: of the words left there, unused)
+            sep_load<S, HAS_AMP>(s, 4 * grp, w, q0);
+            sep_gen<S, HAS_AMP>(q0, gx, gy, f0);
+        }
+        for (int q = 0; q < pad; q += kSepMerge) {
+            const int end = min(q + kSepMerge, pad);
             if constexpr (T == 16) {  // four waves per SIMD overlap by themselves (1.56 against 1.67 ms)
-                for (int e = 0; e < pad; e += S::kStep) {
+                for (int e = q; e < end; e += S::kStep) {
                     sep_load<S, HAS_AMP>(s, e + 4 * grp, w, q0);
                     sep_gen<S, HAS_AMP>(q0, gx, gy, f0);
                     sep_mma<S>(f0, acc);
                 }
             } else {
-                // the operands of a step are formed during the matrix instructions of the step before
-                // (past the last step: of the words left there, unused)
-                sep_load<S, HAS_AMP>(s, 4 * grp, w, q0);
-                sep_gen<S, HAS_AMP>(q0, gx, gy, f0);
-                for (int e = 0; e < pad; e += 2 * S::kStep) {
+                for (int e = q; e < end; e += 2 * S::kStep) {
                     sep_load<S, HAS_AMP>(s, e + S::kStep + 4 * grp, w, q1);
                     sep_gen<S, HAS_AMP>(q1, gx, gy, f1);
                     sep_mma<S>(f0, acc);
@@ -382,21 +437,7 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
                     sep_interleave<S>();
                 }
             }
-        }
-#pragma unroll
-        for (int b = 0; b < NB; ++b) {
-#pragma unroll
-            for (int i = 0; i < R; ++i) {
-#pragma unroll
-                for (int p = 0; p < 2; ++p) {
-                    const float v = sign * (p ? acc.e0[b][p][i] : acc.e0[b][p][i] - npad);
-                    acc.e0[b][p][i] = 0.f;
-                    float sum = o.at(p, b * R + i), cmp = o.at(2 + p, b * R + i);
-                    kahan_add(sum, cmp, v);
-                    o.at(p, b * R + i) = sum;
-                    o.at(2 + p, b * R + i) = cmp;
-                }
-            }
+            merge(sign_of(base + q), end == pad ? npad : 0.f);
         }
     }
     if (!active) return;
@@ -430,10 +471,8 @@ __device__ __forceinline__ void sep_tile(const Geom& g, const double* __restrict
             }
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
-                float sum = o.at(p, b * R + i), cmp = o.at(2 + p, b * R + i);
-                kahan_add(sum, cmp, p ? di : dr);
-                o.at(p, b * R + i) = HAS_AMP ? sum * aback : sum;
-                o.at(2 + p, b * R + i) = HAS_AMP ? cmp * aback : cmp;
+                o.add(p, b * R + i, p ? di : dr);
+                if (HAS_AMP) o.scale(p, b * R + i, aback);
             }
         }
     }
@@ -461,11 +500,12 @@ __global__ __launch_bounds__(kBlock, S::kWaves) void k_fwd_sep(Geom g, const dou
         sep_pixel<S>(tx0, ty0, threadIdx.x >> 6, threadIdx.x & 63, i, x, y);
         if (x < gs.n0 && y < gs.n1) {
             const size_t idx = (size_t)x * gs.n1 + y;
-            if (partial != nullptr)
-                partial[(size_t)blockIdx.y * npix + idx] = make_float4(o.at(0, i), o.at(1, i), o.at(2, i), o.at(3, i));
-            else
-                store_split(gs, x, y, (double)o.at(0, i) - (double)o.at(2, i), (double)o.at(1, i) - (double)o.at(3, i),
-                            out, kind, idx);
+            if (partial != nullptr) {
+                const float2 re = o.parts(0, i), im = o.parts(1, i);
+                partial[(size_t)blockIdx.y * npix + idx] = make_float4(re.x, im.x, re.y, im.y);
+            } else {
+                store_split(gs, x, y, o.value(0, i), o.value(1, i), out, kind, idx);
+            }
         }
     }
 }
@@ -500,8 +540,7 @@ __global__ __launch_bounds__(kBlock, S::kWaves) void k_batched_sep(Geom g0, cons
             int x, y;
             sep_pixel<S>(tx0, ty0, threadIdx.x >> 6, threadIdx.x & 63, i, x, y);
             if (x < gs.n0 && y < gs.n1)
-                store_split(gs, x, y, (double)o.at(0, i) - (double)o.at(2, i), (double)o.at(1, i) - (double)o.at(3, i),
-                            outs, kind, (size_t)x * gs.n1 + y);
+                store_split(gs, x, y, o.value(0, i), o.value(1, i), outs, kind, (size_t)x * gs.n1 + y);
         }
     }
 }
