@@ -15,20 +15,20 @@
 //     + v2 Im [Z20 + i c Z31] + w2 Im [Z02 + i c Z13] + mu Im [Z11 + i c Z22] + nu1 Im Z21 + nu2 Im Z12,
 // (c, e1, e2, k2) = 2 pi (mu, nu1, nu2, ka) . r', with an x^3 in Z as f x, f = <x^4> / <x^2> (its best
 // linear part); mu holds x^3 y and x y^3 in the same way.  The planner bounds what is
-// left out.  Measured against 64 bits over 9 geometries 2.1e-7 .. 3.4e-7 of the gradients (k_adjoint
-// 3.2e-7 .. 4.0e-7).  A square takes 2 T sincos per emitter where k_adjoint takes T^2.
+// left out.  Measured against 64 bits over 9 geometries (64^2 to 2000^2 pixels, even and uneven weights) 1.7e-7 .. 3.0e-7
+// of the gradients (k_adjoint 2.2e-7 .. 4.8e-7).  A square takes 2 T sincos per emitter where k_adjoint takes T^2.
 //
 // Weights and phasors are split into two FP16 parts (T_0, T_1: three products; T_2 and T_3, of second
-// order, the high parts alone), the weights scaled per square by a power of two.  A wave owns a square
+// order, the high parts alone), the weights scaled per square by a power of two (kHalfTop).  A wave owns a square
 // and keeps its weights (of 32 pixels T_2's and T_3's in LDS: they spilled, 812 against 766 us of a
 // gradient at 512^2 x 20000) while the workgroup's 256 emitters pass, T at a time: lane l holds emitter
 // l % T, forms the phasors X of 4 columns per instruction in the operand layout, and after the products
 // its rows y of T_a for that emitter.  The sums over y, the moments and their fold are FP32 (as
 // k_adjoint's sums over 256 pixels); workgroup tiles of 2 x 2 squares are then folded in FP64 as there.
 //
-// Bound by the vector instructions of the sums over y (about 40 per row and emitter; the matrix cores
-// are a third busy).  k_adjoint -> this: 1880 -> 470 us at 512^2 x 20000 with amplitudes (squares of
-// 32), 68 -> 42 us at 256^2 x 4096 (of 16).
+// Bound by the vector instructions of the sums over y (about 40 per row and emitter: 0.40 of the cycles at
+// least, the matrix cores 0.36, 0.35 of the wave cycles wait for an issue slot).  k_adjoint -> this: 1880 -> 430 us at
+// 512^2 x 20000 with amplitudes (squares of 32), 68 -> 42 us at 256^2 x 4096 (of 16).
 #include "mfma_util.hpp"
 #include "adjoint.hpp"
 

@@ -361,8 +361,8 @@ int run_forward_partials(idisim_handle* h, const FwdCall& c, int tile, int split
 
 // The separable tiles take a forward of at least kSepPairs emitter-pixel pairs (n rounded down to its
 // tuning bucket) where they meet the bound.  Intensities: from 1e8 on (1000 emitters on 128 x 128
-// pixels, 1.6e7 pairs, take 13 to 14 us either way; 2048 on 256 x 256, 1.3e8 pairs, 22 against 34 us;
-// 12345 on 333 x 211 79 against 144; 100000 on 512 x 512 1.07 against 3.29 ms).  Fields, of idisim_forward
+// pixels, 1.6e7 pairs, take 13 to 14 us either way; 2048 on 256 x 256, 1.3e8 pairs, 24 against 35 us;
+// 12345 on 333 x 211 80 against 147; 100000 on 512 x 512 1.05 against 3.33 ms).  Fields, of idisim_forward
 // and of idisim_loss_grad_l2 alike: from 5e8 on.  Between the two lines they would be faster as well (4096
 // on 256 x 256: 30 against 52 us); but the FP64 loss of a fit follows its field's rounding (1.3e-7 from 64 bits
 // with these tiles, up to 3.9e-7 with the others), and fits of that size keep the loss that they had.
@@ -1319,7 +1319,7 @@ static int adjoint_call(const char* who, idisim_handle* h, const double* emitter
     const Geom gl = split_geom(h, adj_tile, &w);
     const bool lam = w && !gl.nf;
     // The separable form wherever its squares meet the bound: faster from the smallest sizes on (a call
-    // at 16^2 x 1 34 -> 24 us; the kernel at 256^2 x 4096 68 -> 42 us, at 512^2 x 20000 1880 -> 470).
+    // at 16^2 x 1 34 -> 24 us; the kernel at 256^2 x 4096 68 -> 42 us, at 512^2 x 20000 1880 -> 430).
     // Squares of 32 pixels take 0.6 of the time per pair of those of 16, where their workgroups fill the
     // device.
     const bool want_amp = grad_amp != nullptr;

@@ -102,8 +102,9 @@ __global__ __launch_bounds__(256) void k_chargesharing(const double* __restrict_
 // each output pixel still sums its deposits in the reference's order, with the FP64
 // values of k_chargesharing to rounding, without redrawing a hit for every deposit.
 // Bound by the erf and by the lanes with the most hits around them.  One erf an edge for two a factor:
-// 196 -> 175 us at 512^2, 1e6 photons, sigma 0.75, and 1615 -> 1453 at 900^2, 3e6, sigma 1.6; a whole row of
-// neighbours a loop or smaller chunks were slower where a pixel has many hits (740 -> 926 us).
+// 321 -> 296 us at 512^2, speckle of 1e6 photons, sigma 0.75 (a flat image 196 -> 175), and flat 1615 -> 1453 at
+// 900^2, 3e6, sigma 1.6; a whole row of neighbours a loop or smaller chunks were slower where a pixel has many
+// hits (740 -> 926 us).
 // Dynamic LDS: (16 + 2w)^2 + 1 ints (hit offsets), then cap records of 4w + 3 doubles.
 constexpr int kCsTile = 16;
 

@@ -417,7 +417,8 @@ inline double plan_bound(const Planner* h, int v, double rho)
     }
     if (tile_sep(v)) {
         // a second sincos; the phasors split into two FP16 parts each (2^-23 per component, the product
-        // of the low parts dropped); the mixed terms
+        // of the low parts dropped; with amplitudes of each emitter's own down to 2^-16 of the largest in its
+        // range, below that of 2^-16 of that one); the mixed terms
         const double trunc = sep_trunc(h, v, rho);
         if (!(trunc <= kSepTruncRev)) return std::numeric_limits<double>::infinity();
         e += kSinCosErrRev + trunc + sep_half_error(h, v, rho) + 12.0 * u24 * kInv2Pi;

@@ -15,11 +15,13 @@
 //
 // The sums without a remainder keep FP32's precision: X and Y are formed in FP32 and split into two
 // FP16 parts each (22 bits; X_hi Y_hi + X_hi Y_lo + X_lo Y_hi, the products exact, the sums in FP32).
-// The split by itself costs 7e-8 relative L2.  The remainder's sums are weighted by M and need 1e-3
-// of that: the high parts alone (variant 22, whose M is ten times as large, splits the one along mu).
-// The image of 100000 emitters on 512 x 512 pixels is within 6.9e-7 and 6.8e-7 of 64 bits at two draws
-// (7.5e-7 and 6.1e-7 with the mirror pairs of variant 13), 12345 emitters on 333 x 211 in the far field
-// within 4.6e-7 (6.2e-7).
+// The split by itself costs 7e-8 relative L2, whatever the amplitudes (kHalfTop).  The remainder's sums are
+// weighted by M and need 1e-3 of that: the high parts alone (variant 22, whose M is ten times as large,
+// splits the one along mu).
+// Relative L2 of the field against 64 bits, with the mirror-pair tiles in brackets: 100000 emitters on 512 x 512
+// pixels 3.8e-7 to 4.0e-7 (6.1e-7 to 7.5e-7), 12345 on 333 x 211 in the far field 3.6e-7 (6.3e-7), 64 shots of
+// 1000 to 50000 on 256 x 256 at 0.1 m (variant 22, intensity) 5.9e-7 (1.6e-6), 1e6 with amplitudes on
+// 1024 x 1024 4.3e-7 (3.8e-7).
 //
 // A wave owns one rectangle.  v_mfma_f32_32x32x16_f16 (16x16x32 for T = 16) takes 8 (16) emitters per
 // instruction as K = (re, im) pairs; lane l holds row l % T of X and column l % T of Y for 4 of them,
@@ -27,11 +29,12 @@
 // emitter records (FP64, about the workgroup's centre, once per workgroup of 2 x 2 rectangles) go
 // through LDS.
 //
-// What bounds it: per step of 8 emitters a wave of 32 x 32 pixels issues 66 VALU, 16 transcendental
-// and 10 matrix instructions.  Counters (100000 emitters, 512 x 512): VALU issue 0.79 of the time, the
-// matrix cores 0.5, and the clock at 1.83 GHz (2.24 under the mirror-pair kernel).  That image takes
-// 1.07 ms against 3.29 ms with variant 13.  Sharing X between two blocks of columns (variants 19, 20:
-// one wave per SIMD, 512 registers) saves a quarter of the VALU and 10 to 14% of the time.
+// What bounds it: per step of 8 emitters a wave of 32 x 32 pixels issues 77 vector, 12 transcendental
+// and 10 matrix instructions.  Counters of variant 20 (100000 emitters, 512 x 512): the matrix cores are busy
+// for 0.60 of the cycles and the vector instructions take 0.36 at least; with one wave per SIMD the two
+// hardly overlap, and the clock falls to 1.65 GHz under the counters (2.12 with the mirror-pair kernel).  That image takes
+// 1.05 ms against 3.33 ms with variant 13.  Sharing X between two blocks of columns (variants 19, 20:
+// one wave per SIMD, 512 registers) saves a quarter of the vector instructions and 10% of the time.
 #include "mfma_util.hpp"
 
 namespace idisim {
@@ -187,18 +190,21 @@ __device__ __forceinline__ void sep_mma(const SepFrags<S>& f, SepAcc<S>& acc)
     }
 }
 
-// The matrix instructions of one step spread between the vector instructions of the next: a wave
-// whose matrix instructions follow one another waits for each, and the waves of a SIMD, which start
-// together, do so at the same time (1.20 against 1.07 ms for 100000 emitters on 512 x 512).
+// The matrix instructions of one step spread between the vector instructions of the next, for the shape with the
+// most of them in one wave per SIMD (variant 20: 1.138 against 1.158 ms with amplitudes and 1.094 against
+// 1.100 without, 100000 emitters on 512 x 512); the compiler's own order is better elsewhere (variant 17 with
+// amplitudes 1.140 against 1.164, 18 1.267 against 1.281, 19 1.010 against 1.026).
 template <class S>
 __device__ __forceinline__ void sep_interleave()
 {
-    constexpr int kMma = S::NB * (6 + 2 * S::NE);  // not used with Q2
-    constexpr int kValu = 4 * (8 + S::NE + 10 * S::NB);
+    if constexpr (S::NB == 2 && S::NE == 3) {
+        constexpr int kMma = S::NB * (6 + 2 * S::NE);
+        constexpr int kValu = 4 * (8 + S::NE + 10 * S::NB);
 #pragma unroll
-    for (int i = 0; i < kMma; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x402, kValu / kMma, 0);
+        for (int i = 0; i < kMma; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, kValu / kMma, 0);
+        }
     }
 }
 
