@@ -84,7 +84,12 @@ extern "C" {
                                      sub-block, 15 as 14 with the rotation
                                      between the pair centres also from the
                                      sub-block reference (FP32-split only,
-                                     32x32 px);
+                                     32x32 px); 16 is no variant; 17..22 matrix
+                                     products over the emitters (FP32-split only,
+                                     not with sum mode 1; 64x64, 64x64, 64x128,
+                                     64x128, 32x32, 32x32 px), the remainder along
+                                     two directions (17, 19, 21), in full (18, 20)
+                                     or to second order (22);
                                      FP64 handles take 0..3                      */
 #define IDISIM_OPT_SPLIT        3 /* force emitter split count (0 = planner)        */
 #define IDISIM_OPT_SUMMODE      4 /* 0 (default): per-chunk partials merged with
