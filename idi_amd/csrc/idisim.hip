@@ -837,7 +837,7 @@ int idisim_create(idisim_handle** out, const idisim_geometry* geom, int precisio
         h->num_cus = prop.multiProcessorCount;
     h->g = make_geom(*geom);
     planner_tables(h);
-    planner_sep_tables(h);
+    if (precision == IDISIM_PREC_FP32SPLIT) planner_sep_tables(h);  // no FP64 call takes a separable tile
     h->plan.precision = precision;
     if (hipHostMalloc(reinterpret_cast<void**>(&h->h_viol), sizeof(unsigned int),
                       hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
