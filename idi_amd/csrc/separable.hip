@@ -210,7 +210,7 @@ __device__ __forceinline__ void sep_interleave()
 
 // The long sums of a lane's pixels, word i = b R + register of block b, part p (re, im).  T = 16: FP32 with
 // compensations in registers; T = 32: FP64 in LDS, added to without reading them back (ds_add_f64; four
-// words read, compensated and written cost 1.151 against 1.040 ms for 100000 emitters on 512 x 512).
+// words read, compensated and written cost 1.151 against 1.053 ms for 100000 emitters on 512 x 512).
 template <class S>
 struct SepOut {
     static constexpr int N = S::NB * S::R;
